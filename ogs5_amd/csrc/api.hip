@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "kernels.hpp"
+#include "resident.hpp"
 #include "ogsx_internal.h"
 
 using namespace ogsx;
@@ -41,23 +42,19 @@ int fail(int code, const std::string& msg)
 
 // Blocks of the n-sized kernels of one system (each block a contiguous chunk
 // of rows).  G sets the partial-sum layout, so it is a function of n alone,
-// never tuned at run time: one row per thread up to OGSX_FILL_BLOCKS blocks,
-// then OGSX_ROWS_PER_BLOCK rows per block, at most kMaxGrid (2048) blocks
-// (the partial sums' reduction loads all of them in one batch).
-// Few rows per block keep mid-size systems (latency-bound) spread over the
-// CUs; many rows per block cut block dispatches and the per-block reduction
-// of partial sums for large systems and for groups of many systems.
+// never tuned at run time: one row per thread up to kResMaxRows rows (the
+// systems that resident launches hold on the chip, a thread per row), then
+// OGSX_ROWS_PER_BLOCK rows per block, at most kMaxGrid (2048) blocks (the
+// partial sums' reduction loads all of them in one batch).  Many rows per
+// block cut block dispatches and the per-block reduction of partial sums.
 #ifndef OGSX_ROWS_PER_BLOCK
 #define OGSX_ROWS_PER_BLOCK 1024
-#endif
-#ifndef OGSX_FILL_BLOCKS
-#define OGSX_FILL_BLOCKS 256
 #endif
 
 int grid_for(int64_t n)
 {
-    int64_t g = (n + OGSX_ROWS_PER_BLOCK - 1) / OGSX_ROWS_PER_BLOCK;
-    g = std::max<int64_t>(g, std::min<int64_t>((n + kBlock - 1) / kBlock, OGSX_FILL_BLOCKS));
+    int64_t g = n <= kResMaxRows ? (n + kBlock - 1) / kBlock
+                                 : (n + OGSX_ROWS_PER_BLOCK - 1) / OGSX_ROWS_PER_BLOCK;
     g = (g + kNumXcd - 1) / kNumXcd * kNumXcd;
     return (int)std::max<int64_t>(kNumXcd, std::min<int64_t>(g, kMaxGrid));
 }
@@ -140,6 +137,9 @@ struct SolveCtx {
     int total = 0, updates = 0;
     int converged = 0, ret = 0;
     double error = 0.0, bnorm = 0.0;
+    // batches still to run as separate launches after a resident launch had
+    // to leave, and how often that happened (kResMaxLeaves: no further try)
+    int res_wait = 0, res_leaves = 0;
     // convergence rate of the running recurrence segment, for batch sizing
     int seg_key = -1, seg_it0 = 0;
     double seg_e0 = 0.0;
@@ -217,7 +217,8 @@ struct ogsx_system {
     DevVecs<double> v64;
     DevVecs<float> v32;
     double* r64 = nullptr;  // IR residual
-    double* part = nullptr; // partial sums [4][G] x 3 sets
+    double* part = nullptr; // partial sums: 16 x part_stride(G)
+    ResSync* rs = nullptr;  // exchange buffers of resident launches
     double* red = nullptr;  // reduced scalars
     KrylovState* st = nullptr;
     // device descriptor of this system and its per-solve parameters
@@ -704,7 +705,8 @@ int64_t system_bytes(const ogsx_pattern* p, int precision)
     const int ed = edim_of(h.etype);
     int64_t t = b(n + 1, 4) + b(nnz, 4) + b(n, 4) + b((int64_t)h.conn.size(), 4) +
                 b((int64_t)h.color_elems.size(), 4) + b((int64_t)h.conn.size() * h.npe, 4) + b(nnz, 8) +
-                2 * b(n, 8) + 12 * b(n, 8) + b(16 * G, 8) + b(8, 8) + b(1, sizeof(KrylovState)) +
+                2 * b(n, 8) + 12 * b(n, 8) + b(16 * (int64_t)part_stride((int)G), 8) +
+                b((int64_t)res_sync_bytes((int)G), 1) + b(8, 8) + b(1, sizeof(KrylovState)) +
                 b(n, 1) + b(n, 8) + b(1, sizeof(SysDev)) + b(1, sizeof(KrylovParams));
     if (precision == OGSX_FP32_IR) t += b(nnz, 4) + 12 * b(n, 4) + b(n, 8) + b(1, sizeof(IRState));
     if (!L.sell16)  // tiles and 32-bit SELL columns, built at creation only then
@@ -1091,7 +1093,8 @@ int ogsx_system_create(const ogsx_pattern* p, int precision, ogsx_system** out)
         (rc = dalloc(s, &s->slot, h.conn.size() * h.npe)) || (rc = dalloc(s, &s->A, h.nnz)) ||
         (rc = dalloc(s, &s->uold, h.n)) || (rc = dalloc(s, &s->ic, h.n)) ||
         (rc = alloc_vecs(s, s->v64)) ||
-        (rc = dalloc(s, &s->part, (size_t)16 * s->G)) || (rc = dalloc(s, &s->red, 8)) ||
+        (rc = dalloc(s, &s->part, 16 * part_stride(s->G))) ||
+        (rc = dalloc(s, (char**)&s->rs, res_sync_bytes(s->G))) || (rc = dalloc(s, &s->red, 8)) ||
         (rc = dalloc(s, &s->st, 1)) || (rc = dalloc(s, &s->bcflag, h.n)) ||
         (rc = dalloc(s, &s->bcg, h.n)))
         return cleanup(rc);
@@ -1125,6 +1128,8 @@ int ogsx_system_create(const ogsx_pattern* p, int precision, ogsx_system** out)
     double* zv[] = {s->v64.x, s->v64.b, s->uold, s->ic};
     for (double* q : zv) k_fill<double><<<blocks_for(h.n, kBlock * 4), kBlock, 0, s->stream>>>(h.n, q, 0.0);
     k_fill<int8_t><<<blocks_for(h.n, kBlock * 4), kBlock, 0, s->stream>>>(h.n, s->bcflag, (int8_t)0);
+    k_res_clear<<<blocks_for(res_slot_count(s->G), kBlock), kBlock, 0, s->stream>>>(
+        s->rs, res_slot_count(s->G));
     if (hipStreamSynchronize(s->stream) != hipSuccess || hipGetLastError() != hipSuccess)
         return cleanup(fail(OGSX_EHIP, "initialisation kernels failed"));
     s->lay = &p->L;
@@ -1208,6 +1213,7 @@ int ogsx_system_create(const ogsx_pattern* p, int precision, ogsx_system** out)
         d.part = s->part;
         d.red = s->red;
         d.st = s->st;
+        d.rs = s->rs;
         d.prm = s->prm;
         d.irs = s->irs;
         d.n = s->n;

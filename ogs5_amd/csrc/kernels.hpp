@@ -50,6 +50,18 @@ __device__ __forceinline__ void chunk_of(int n, int G, int b, int& beg, int& end
     end = (int)((int64_t)n * (c + 1) / G);
 }
 
+// Rows of block b: its chunk of 64-row slices.  Every kernel that sums over
+// rows -- SpMV and vector kernels of every format, and the resident kernels
+// -- uses this split, thread t taking rows beg + t + 256 j in that order, so
+// a dot product rounds the same whichever of them computes it.
+__device__ __forceinline__ void row_chunk(int n, int G, int b, int& beg, int& end)
+{
+    int sb, se;
+    chunk_of((n + 63) / 64, G, b, sb, se);
+    beg = sb * 64;
+    end = min(se * 64, n);
+}
+
 __device__ __forceinline__ double wave_sum(double v)
 {
 #pragma unroll
@@ -57,7 +69,22 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
-// Block-reduces NV values and stores them as partials[k*G + b].
+// Partial sums of one dot product: one per block, in the order of the
+// blocks' rows (chunk c = block b's chunk index).  They are added q = 1, 2, 4
+// or 8 neighbours at a time (thread t: chunks q t .. q t + q - 1, in order),
+// then over the 256 threads' wave and block sums -- a workgroup that works
+// on q neighbouring chunks can add their partials itself and hand on one
+// value, with the same rounding.  Chunk c is stored at 256 (c % q) + c / q,
+// so thread t's j-th partial is at 256 j + t.
+constexpr int kMaxGrid = 2048;
+__host__ __device__ constexpr int part_q(int G)
+{
+    return G <= kBlock ? 1 : G <= 2 * kBlock ? 2 : G <= 4 * kBlock ? 4 : 8;
+}
+// Doubles per dot product in the partial-sum buffer.
+__host__ __device__ constexpr size_t part_stride(int G) { return (size_t)kBlock * part_q(G); }
+
+// Block-reduces NV values and stores them as partials of block b.
 template <int NV>
 __device__ __forceinline__ void store_partials(double (&v)[NV], OGSX_GL double* partials, int G,
                                                int b)
@@ -71,46 +98,49 @@ __device__ __forceinline__ void store_partials(double (&v)[NV], OGSX_GL double* 
     }
     __syncthreads();
     if (threadIdx.x == 0) {
+        const int c = (b % kNumXcd) * (G / kNumXcd) + b / kNumXcd;
+        const int q = part_q(G);
+        OGSX_GL double* at = partials + kBlock * (c % q) + c / q;
 #pragma unroll
         for (int k = 0; k < NV; k++) {
             double s = sm[k][0];
 #pragma unroll
             for (int w = 1; w < kBlock / 64; w++) s += sm[k][w];
-            partials[(size_t)k * G + b] = s;
+            at[k * part_stride(G)] = s;
         }
     }
 }
 
 // Sums G partials per value in a fixed order; every thread gets the result.
 // G is the grid size of the producer, which equals this kernel's grid, and
-// at most kMaxGrid (grid_for's cap).  Thread t adds partials t, t + kBlock,
-// t + 2 kBlock, ... in that order, all loaded before the first add, so a
-// block waits for one round trip to L2 instead of one per partial (the
-// partials were written by blocks on every XCD and miss the local L2).
-constexpr int kMaxGrid = 2048;
+// at most kMaxGrid (grid_for's cap).  A thread's partials are all loaded
+// before the first add, so a block waits for one round trip to L2 instead of
+// one per partial (the partials were written by blocks on every XCD and miss
+// the local L2).
 constexpr int kPartialBatch = kMaxGrid / kBlock;
 template <int NV>
 struct PartialLoads {
     double t[NV][kPartialBatch];
 };
 
-// The first kPartialBatch partials per value of thread t, loaded (not yet
-// added).  A kernel that also streams rows issues these loads first and its
-// rows' loads after them, so that the reduction can wait for the partials
-// (from L2) while the rows (from HBM) are still in flight: a wait on the
-// memory counter covers every load issued before the one awaited.
+// The partials of thread t, loaded (not yet added).  A kernel that also
+// streams rows issues these loads first and its rows' loads after them, so
+// that the reduction can wait for the partials (from L2) while the rows
+// (from HBM) are still in flight: a wait on the memory counter covers every
+// load issued before the one awaited.
 template <int NV>
 __device__ __forceinline__ void load_partials(const OGSX_GL double* partials, int G,
                                               PartialLoads<NV>& P)
 {
+    const int q = part_q(G), t = threadIdx.x;
 #pragma unroll
     for (int k = 0; k < NV; k++)
 #pragma unroll
         for (int j = 0; j < kPartialBatch; j++) {
-            // clamped index: every load is issued unpredicated (G >= 1)
-            const int i = threadIdx.x + j * kBlock;
-            const double x = partials[(size_t)k * G + (i < G ? i : G - 1)];
-            P.t[k][j] = i < G ? x : 0.0;
+            // clamped index: every load is issued unpredicated
+            const bool have = j < q && q * t + j < G;
+            const double x = partials[k * part_stride(G) + (have ? kBlock * j + t : 0)];
+            P.t[k][j] = have ? x : 0.0;
         }
 }
 
@@ -194,7 +224,7 @@ template <typename Body>
 __device__ __forceinline__ void vec_chunk(int n, int G, int b, Body&& body)
 {
     int beg, end;
-    chunk_of(n, G, b, beg, end);
+    row_chunk(n, G, b, beg, end);
     for (int i = beg + threadIdx.x; i < end; i += kBlock) body(i);
 }
 
@@ -215,7 +245,7 @@ __device__ __forceinline__ bool vec_chunk_batched_mid(int n, int G, int b, Load&
                                                       Apply&& apply)
 {
     int beg, end;
-    chunk_of(n, G, b, beg, end);
+    row_chunk(n, G, b, beg, end);
     const int last = end - 1;
     int i = beg + threadIdx.x;
     if (i < end) {
@@ -762,9 +792,8 @@ __device__ __forceinline__ void spmv_crs1(const GMat<VT>& m, const OGSX_GL XT* _
                                           int G, int b, Epi&& epi)
 {
 #pragma clang fp contract(off)
-    int sb, se;
-    chunk_of((m.n + kSellC - 1) / kSellC, G, b, sb, se);
-    const int beg = sb * kSellC, end = min(se * kSellC, m.n);
+    int beg, end;
+    row_chunk(m.n, G, b, beg, end);
     for (int r = beg + (int)threadIdx.x; r < end; r += kBlock) {
         const int k1 = m.ptr[r + 1];
         ACC s = 0;
@@ -793,7 +822,7 @@ __device__ __forceinline__ void spmv_symdia_k(const GMat<VT>& m, const OGSX_GL X
                                               int G, int b, Epi&& epi)
 {
     int beg, end;
-    chunk_of(m.n, G, b, beg, end);
+    row_chunk(m.n, G, b, beg, end);
     const int n = m.n, K = KC > 0 ? KC : m.dia_k;
     const OGSX_GL VT* dv = m.dia_val;
     // R rows per thread at a time (i, i + kBlock, ...; those past the chunk
@@ -846,9 +875,8 @@ __device__ __forceinline__ void spmv_symdia_crs_k(const GMat<VT>& m, const OGSX_
     // the rows of its chunk of 64-row slices, thread t the rows R0 + t +
     // 256 j in that order), so the solve kernels' fused dot products round
     // as with those formats
-    int sb, se;
-    chunk_of((m.n + kSellC - 1) / kSellC, G, b, sb, se);
-    const int beg = sb * kSellC, end = min(se * kSellC, m.n);
+    int beg, end;
+    row_chunk(m.n, G, b, beg, end);
     const int n = m.n, K = KC > 0 ? KC : m.dia_k;
     const OGSX_GL VT* dv = m.dia_val;
     // one row per thread at a time: two (the FP32 form's) took 229 VGPRs
@@ -1656,6 +1684,7 @@ struct KrylovParams {
     int ir_reliable;      // 1 reliable-update CG, 0 restarted refinement
     int ir_scaled;        // 1: the FP32 recurrence runs on S A S with
                           // S = diag(1/sqrt|a_ii|) (single-reduction CG)
+    int dia;              // the FP64 matrix is read from its symmetric diagonal copy
 };
 
 // Refinement state of an IR solve, advanced by k_ir_decide.
@@ -1672,6 +1701,8 @@ struct IRState {
     int pad;
 };
 
+struct ResSync;
+
 struct SysDev {
     MatView<double> m64;
     MatView<float> m32;
@@ -1686,11 +1717,12 @@ struct SysDev {
     const int* tri_src;  // CRS position of every slice-triple entry (-1 = zero)
     const int* dia_src;  // ... of every symmetric-diagonal entry (-1 = zero)
     double* r64;         // IR residual
-    double* part;        // partial sums [16][G]
+    double* part;        // partial sums [16][part_stride(G)]
     double* red;         // reduced scalars
     KrylovState* st;
     KrylovParams* prm;
     IRState* irs;        // IR systems
+    ResSync* rs;         // exchange buffers of resident launches (resident.hpp)
     int n, G, nnz, npad, npad3;
 };
 
@@ -1998,7 +2030,7 @@ __device__ __forceinline__ void cg_update_body(const Grp& g, int vb)
     const OGSX_GL T* __restrict__ d = v.d;
     const int b = c.b;
     int beg, end;
-    chunk_of(S.n, c.G, b, beg, end);
+    row_chunk(S.n, c.G, b, beg, end);
     constexpr int U = 4;
     int i = beg + threadIdx.x;
     // the first batch of the stream does not depend on alpha: its loads are
@@ -2103,7 +2135,7 @@ __device__ __forceinline__ void cg_update_body(const Grp& g, int vb)
             acc[0] += (double)rn * (double)rn;
             acc[1] += (double)zi * (double)rn;
         }
-        store_partials<2>(acc, gl(S.part) + 4 * (size_t)c.G, c.G, b);
+        store_partials<2>(acc, gl(S.part) + 4 * part_stride(c.G), c.G, b);
     }
     if (c.b == 0 && threadIdx.x == 0) {
         st->rr_old = rr;
@@ -2133,12 +2165,12 @@ __device__ __forceinline__ void cg_direction_body(const Grp& g, int vb)
     const OGSX_GL T* __restrict__ r = v.r;
     const OGSX_GL T* __restrict__ d = v.d;
     int beg, end;
-    chunk_of(S.n, c.G, c.b, beg, end);
+    row_chunk(S.n, c.G, c.b, beg, end);
     constexpr int U = 4;
     int i = beg + threadIdx.x;
     // first batch loaded before the reduction (independent of beta)
     PartialLoads<2> pl;  // partials first, then the first batch of rows
-    load_partials<2>(gl(S.part) + 4 * (size_t)c.G, c.G, pl);
+    load_partials<2>(gl(S.part) + 4 * part_stride(c.G), c.G, pl);
     T pi[U], ri[U], di[U];
     const bool first = i + (U - 1) * kBlock < end;
     // the extra row of a chunk of 1024-1280 rows, as in the update
@@ -2168,7 +2200,7 @@ __device__ __forceinline__ void cg_direction_body(const Grp& g, int vb)
         }
     }
     double s[2];
-    finish_partials<2>(gl(S.part) + 4 * (size_t)c.G, c.G, pl, s);
+    finish_partials<2>(gl(S.part) + 4 * part_stride(c.G), c.G, pl, s);
     const double rnorm = sqrt(s[0]);
     const double error = rnorm / st->bnorm;
     const double tol = gl(S.prm)->tol;
@@ -2239,7 +2271,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_rescan(Grp g)
             acc[0] += (double)ri * (double)ri;
             acc[1] += (double)zi * (double)ri;
         });
-        store_partials<2>(acc, gl(S.part) + 4 * (size_t)c.G, c.G, b);
+        store_partials<2>(acc, gl(S.part) + 4 * part_stride(c.G), c.G, b);
     }
 }
 
@@ -2252,7 +2284,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_resume(Grp g)
     const SysDev& S = *c.S;
     if (skip_action(S, 2)) return;
     double s[2];
-    reduce_partials<2>(gl(S.part) + 4 * (size_t)c.G, c.G, s);
+    reduce_partials<2>(gl(S.part) + 4 * part_stride(c.G), c.G, s);
     OGSX_GL KrylovState* st = gl(S.st);
     const T beta = (T)(s[1] / st->rr_old);
     const GVec<T> v = gvec(kv_of<T>(S));
@@ -2420,7 +2452,7 @@ __device__ __forceinline__ void bi_spmv_v_body(const Grp& g, int vb)
             v.v[i] = ax;
             acc[0] += (double)v.r0[i] * (double)ax;
         });
-        store_partials<1>(acc, gl(S.part) + 4 * (size_t)c.G, c.G, b);
+        store_partials<1>(acc, gl(S.part) + 4 * part_stride(c.G), c.G, b);
     }
     if (c.b == 0 && threadIdx.x == 0) st->iter = st->iter + 1;
 }
@@ -2440,7 +2472,7 @@ __device__ __forceinline__ void bi_s_body(const Grp& g, int vb)
     OGSX_GL KrylovState* st = gl(S.st);
     if (st->done || st->pend) return;
     PartialLoads<1> pl;  // partials first, then the first batch of rows
-    load_partials<1>(gl(S.part) + 4 * (size_t)c.G, c.G, pl);
+    load_partials<1>(gl(S.part) + 4 * part_stride(c.G), c.G, pl);
     const double rho1 = st->rho1;
     double alpha_d = 0.0;
     T alpha = 0;
@@ -2458,7 +2490,7 @@ __device__ __forceinline__ void bi_s_body(const Grp& g, int vb)
             },
             [&]() -> bool {
                 double sv[1];
-                finish_partials<1>(gl(S.part) + 4 * (size_t)c.G, c.G, pl, sv);
+                finish_partials<1>(gl(S.part) + 4 * part_stride(c.G), c.G, pl, sv);
                 alpha_d = rho1 / sv[0];
                 alpha = (T)alpha_d;
                 return true;
@@ -2469,7 +2501,7 @@ __device__ __forceinline__ void bi_s_body(const Grp& g, int vb)
                 v.sh[k] = si / dd[u];
                 acc[0] += (double)si * (double)si;
             });
-        store_partials<1>(acc, gl(S.part) + 8 * (size_t)c.G, c.G, b);
+        store_partials<1>(acc, gl(S.part) + 8 * part_stride(c.G), c.G, b);
     }
     if (c.b == 0 && threadIdx.x == 0) {
         st->alpha = alpha_d;
@@ -2493,7 +2525,7 @@ __device__ __forceinline__ void bi_spmv_t_body(const Grp& g, int vb)
     OGSX_GL KrylovState* st = gl(S.st);
     if (st->done || st->pend) return;
     double ss[1];
-    reduce_partials<1>(gl(S.part) + 8 * (size_t)c.G, c.G, ss);
+    reduce_partials<1>(gl(S.part) + 8 * part_stride(c.G), c.G, ss);
     const double err = sqrt(ss[0]) / st->bnorm;
     const GVec<T> v = gvec(kv_of<T>(S));
     if (err < gl(S.prm)->tol) {
@@ -2514,7 +2546,7 @@ __device__ __forceinline__ void bi_spmv_t_body(const Grp& g, int vb)
             acc[0] += (double)ax * (double)ax;
             acc[1] += (double)ax * (double)v.s[i];
         });
-        store_partials<2>(acc, gl(S.part) + 12 * (size_t)c.G, c.G, b);
+        store_partials<2>(acc, gl(S.part) + 12 * part_stride(c.G), c.G, b);
     }
 }
 
@@ -2534,7 +2566,7 @@ __device__ __forceinline__ void bi_update_body(const Grp& g, int vb)
     OGSX_GL KrylovState* st = gl(S.st);
     if (st->done || st->pend) return;
     PartialLoads<2> pl;  // partials first, then the first batch of rows
-    load_partials<2>(gl(S.part) + 12 * (size_t)c.G, c.G, pl);
+    load_partials<2>(gl(S.part) + 12 * part_stride(c.G), c.G, pl);
     double omega_d = 0.0;
     T omega = 0;
     const T alpha = (T)st->alpha;
@@ -2555,7 +2587,7 @@ __device__ __forceinline__ void bi_update_body(const Grp& g, int vb)
             },
             [&]() -> bool {
                 double sv[2];
-                finish_partials<2>(gl(S.part) + 12 * (size_t)c.G, c.G, pl, sv);
+                finish_partials<2>(gl(S.part) + 12 * part_stride(c.G), c.G, pl, sv);
                 omega_d = (sv[0] > DBL_MIN) ? sv[1] / sv[0] : 1.0;
                 omega = (T)omega_d;
                 return true;
@@ -3021,7 +3053,7 @@ __device__ __forceinline__ void cg1_update_body(const Grp& g, int vb)
     OGSX_GL T* __restrict__ sv = v.s;
     const OGSX_GL T* __restrict__ w = v.z;
     int beg, end;
-    chunk_of(S.n, c.G, c.b, beg, end);
+    row_chunk(S.n, c.G, c.b, beg, end);
     constexpr int U = 4;
     int i = beg + threadIdx.x;
     // the first batch of the stream does not depend on the scalars: its
@@ -3141,7 +3173,7 @@ __global__ __launch_bounds__(kBlock) void k_cg1_resume(Grp g)
         v.s[i] = sn;
         acc[0] += (double)pn * (double)sn;
     });
-    store_partials<1>(acc, gl(S.part) + 4 * (size_t)c.G, c.G, c.b);
+    store_partials<1>(acc, gl(S.part) + 4 * part_stride(c.G), c.G, c.b);
     if (c.b == 0 && threadIdx.x == 0) st->rr = gamma;
 }
 
@@ -3155,7 +3187,7 @@ __global__ __launch_bounds__(kBlock) void k_cg1_resume_step(Grp g)
     if (skip_action(S, 2)) return;
     OGSX_GL KrylovState* st = gl(S.st);
     double red[1];
-    reduce_partials<1>(gl(S.part) + 4 * (size_t)c.G, c.G, red);
+    reduce_partials<1>(gl(S.part) + 4 * part_stride(c.G), c.G, red);
     const double gamma = st->rr;
     const double alpha_d = gamma / red[0];
     const T alpha = (T)alpha_d;

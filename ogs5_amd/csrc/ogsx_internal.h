@@ -102,7 +102,10 @@ struct KrylovState {
     double sr_gam;    // (r,r) of the iterate the last update started from
     double sr_alp;    // alpha of the last update
     int sr_it;        // iterations completed (>= iter)
-    int sr_pad;
+    int resident;     // last resident launch: 0 ran, 1 left at its census
+                      // (nothing done), 2 a wait ran out (resident.hpp)
+    int row_max;      // longest row (zero-allocation solve only)
+    int pad;
 };
 
 }  // namespace ogsx

@@ -1,0 +1,416 @@
+// resident.hpp -- Krylov iterations in one launch, the system on the chip.
+//
+// A system of up to a few hundred thousand rows spends a Krylov iteration in
+// the dispatch of its three (CG) or five (BiCGStab) dependent launches: on
+// 200 x 200 quads each takes 3.5-4 us, of which the work itself is well
+// under one.  A resident launch keeps one workgroup per few row chunks on
+// the chip for a whole batch of iterations; a thread owns one row and holds
+// its matrix entries, its x, r, p and the direction values of its columns in
+// registers.  What the workgroups exchange -- one double per chunk and dot
+// product, and one vector entry per row -- goes through relaxed agent-scope
+// atomics (sc1 accesses: stores written through, loads served past the
+// non-coherent caches), so no barrier writes back or invalidates an L2: a
+// release / acquire pair per barrier costs 10 us over 256 workgroups, an
+// exchange by atomics 1.4-2.0 us.
+//
+// The exchange of a dot product is also the barrier: every workgroup posts
+// its partial sums and waits for those of all others.  A CG iteration needs
+// two of them.  z = r / d is published before the second, and each thread
+// forms p = z + beta p for its own columns from the z it gathers and the p
+// it kept, so the new direction needs no barrier of its own.
+//
+// Arithmetic: rows, threads, partial sums and their order of addition are
+// those of the separate launches (row_chunk, store_partials,
+// finish_partials), so iterates agree with them bit for bit.
+//
+// Waiting: a launch first counts its workgroups in (res_census).  Only when
+// all of them are resident does any of them enter the iterations; when that
+// takes too long (another launch holds the chip) all leave, nothing has
+// changed, and the host takes the separate launches.  After the census every
+// workgroup runs until the batch ends, so each wait is for a workgroup that
+// is running; the waits are bounded all the same.
+#pragma once
+
+#include "kernels.hpp"
+
+namespace ogsx {
+
+// A slot that holds no partial sum yet: a NaN no dot product yields (a sum
+// with these bits is posted as the default NaN).
+constexpr unsigned long long kSlotEmpty = 0xFFF8DEADBEEF0001ull;
+constexpr int kSlotSets = 3;    // rotating sets of slots
+constexpr int kSlotVals = 3;    // values of one exchange
+// Copies of each slot: workgroup w reads copy w % 8, so that a line is
+// polled by an eighth of the workgroups (256 workgroups: 3.2 -> 2.0 us per
+// exchange; 16: 1.5 -> 1.4 us).
+constexpr int kSlotCopies = 8;
+constexpr int kResMaxSlots = kBlock;          // slots per value and copy
+constexpr int kResMaxRows = 1 << 18;          // rows of a resident system
+constexpr unsigned kResPolls = 1u << 21;      // polls of one wait (seconds)
+constexpr long long kCensusTicks = 20000;     // 100 MHz: 200 us
+constexpr int kCensusRing = 64;
+
+// Exchange buffers of one system, kept between launches.
+struct ResSync {
+    int phase;  // set of the next exchange (its slots are empty)
+    int pad[31];
+    unsigned long long slot[1];  // [set][value][copy][slots]
+};
+
+__host__ __device__ constexpr int res_slots(int G)
+{
+    return ((G + part_q(G) - 1) / part_q(G) + 15) / 16 * 16;
+}
+__host__ __device__ constexpr size_t res_slot_count(int G)
+{
+    return (size_t)kSlotSets * kSlotVals * kSlotCopies * res_slots(G);
+}
+constexpr size_t res_sync_bytes(int G) { return sizeof(int) * 32 + 8 * res_slot_count(G); }
+
+// Arrival count and decision of one launch (0 open, 1 go, 2 leave).
+struct ResCensus {
+    unsigned arrived;
+    int decision;
+    int pad[14];
+};
+
+// One resident launch: its census entry, workgroups in all and iterations.
+struct ResLaunch {
+    ResCensus* ring;
+    int entry;
+    int wgs;
+    int iters;
+};
+
+template <typename T>
+__device__ __forceinline__ T agent_load(const OGSX_GL T* p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void agent_store(OGSX_GL T* p, T v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// A pointer that is the same for the whole wave, kept in scalar registers (a
+// pointer read from a descriptor is not known to be, and each of a thread's
+// gathers would hold a 64-bit address of its own).
+template <typename T>
+__device__ __forceinline__ OGSX_GL T* wave_uniform(OGSX_GL T* p)
+{
+    const unsigned long long v = (unsigned long long)p;
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+    return (OGSX_GL T*)(((unsigned long long)hi << 32) | lo);
+}
+// The wave's loads have returned and its stores have reached the memory that
+// other workgroups read.
+__device__ __forceinline__ void wait_memory() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// Empties the exchange buffers and the phase.
+__global__ __launch_bounds__(kBlock) void k_res_clear(ResSync* rs, size_t count)
+{
+    for (size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x; i < count;
+         i += (size_t)gridDim.x * kBlock)
+        rs->slot[i] = kSlotEmpty;
+    if (blockIdx.x == 0 && threadIdx.x == 0) rs->phase = 0;
+}
+
+// Counts the launch's workgroups in; true when all of them are resident.  A
+// workgroup that has nothing to do (its solve stopped earlier) only counts.
+__device__ __forceinline__ bool res_census(const ResLaunch& L, bool idle, int* flag)
+{
+    // the workgroup has read the state before it counts: another may end the
+    // batch, and write the state, once all have counted
+    wait_memory();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        OGSX_GL ResCensus* c = (OGSX_GL ResCensus*)(L.ring + L.entry);
+        const unsigned before =
+            __hip_atomic_fetch_add(&c->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        int d = 0;
+        auto decide = [&](int want) {
+            int open = 0;
+            const bool mine = __hip_atomic_compare_exchange_strong(
+                &c->decision, &open, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                __HIP_MEMORY_SCOPE_AGENT);
+            d = mine ? want : open;
+        };
+        if (before + 1 == (unsigned)L.wgs) {
+            decide(1);
+        } else if (!idle) {
+            const long long t0 = wall_clock64();
+            for (unsigned polls = 0; d == 0; polls++) {
+                d = agent_load(&c->decision);
+                if (d == 0 && (wall_clock64() - t0 > kCensusTicks || polls > kResPolls)) decide(2);
+            }
+        }
+        if (blockIdx.x == 0) {  // an entry no launch uses now, for a later one
+            OGSX_GL ResCensus* f =
+                (OGSX_GL ResCensus*)(L.ring + (L.entry + kCensusRing / 2) % kCensusRing);
+            agent_store(&f->arrived, 0u);
+            agent_store(&f->decision, 0);
+        }
+        *flag = d == 1;
+    }
+    __syncthreads();
+    return *flag != 0 && !idle;
+}
+
+// Exchange of NV dot products among the workgroups of one system (VB chunks
+// of 256 threads each per workgroup, q chunks to a slot).
+template <int VB>
+struct ResExchange {
+    OGSX_GL unsigned long long* slot;
+    int slots, q, w, set, nwg;
+    double (*sw)[4 * VB];  // [kSlotVals] wave sums
+    double (*sm)[4];       // [kSlotVals] sums of the waves that poll
+    int* ok;
+
+    __device__ __forceinline__ OGSX_GL unsigned long long* at(int s, int k, int copy) const
+    {
+        return slot + ((size_t)(s * kSlotVals + k) * kSlotCopies + copy) * slots;
+    }
+
+    template <int NV>
+    __device__ __forceinline__ bool sum(const double (&v)[NV], double (&out)[NV])
+    {
+        const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+        const int per = VB / q;  // slots this workgroup posts per value
+#pragma unroll
+        for (int k = 0; k < NV; k++) {
+            const double s = wave_sum(v[k]);
+            if (lane == 0) sw[k][wave] = s;
+        }
+        wait_memory();  // vector entries published before this exchange
+        __syncthreads();
+        const int copy = t % kSlotCopies, j = t / kSlotCopies % per, kk = t / kSlotCopies / per;
+        if (kk < NV) {
+            double s = 0.0;
+            for (int i = 0; i < q; i++) {
+                const double* c = &sw[kk][4 * (j * q + i)];
+                s += ((c[0] + c[1]) + c[2]) + c[3];
+            }
+            unsigned long long bits = (unsigned long long)__double_as_longlong(s);
+            if (bits == kSlotEmpty) bits = 0x7FF8000000000000ull;
+            agent_store(at(set, kk, copy) + w * per + j, bits);
+        }
+        if (wave < 4) {
+            unsigned long long got[NV];
+#pragma unroll
+            for (int k = 0; k < NV; k++) got[k] = 0;
+            if (t < nwg * per) {
+                unsigned polls = 0;
+#pragma nounroll
+                for (bool wait = true; wait;) {
+                    wait = false;
+#pragma unroll
+                    for (int k = 0; k < NV; k++) got[k] = agent_load(at(set, k, w % kSlotCopies) + t);
+#pragma unroll
+                    for (int k = 0; k < NV; k++) wait = wait || got[k] == kSlotEmpty;
+                    if (wait && ++polls > kResPolls) {
+                        *ok = 0;
+                        break;
+                    }
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < NV; k++) {
+                const double s = wave_sum(__longlong_as_double((long long)got[k]));
+                if (lane == 0) sm[k][wave] = s;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < NV; k++) out[k] = ((sm[k][0] + sm[k][1]) + sm[k][2]) + sm[k][3];
+        // every workgroup has read the previous set: empty this one's slots
+        // there (it is used again two exchanges on)
+        const int prev = set == 0 ? kSlotSets - 1 : set - 1;
+        if (t < kSlotVals * per * kSlotCopies)
+            agent_store(at(prev, t / kSlotCopies / per, copy) + w * per + j, kSlotEmpty);
+        set = set == kSlotSets - 1 ? 0 : set + 1;
+        return *ok != 0;
+    }
+};
+
+// A row's entries in the order of its sum, padded to NE with zeros: the CRS
+// row, or the symmetric diagonal copy -- in CRS column order (FP64), or as
+// spmv_symdia_k takes it (FP32, PAIR: the diagonal, then each offset's upper
+// and lower entry).  col holds byte offsets into a T vector.
+template <typename T, int NE, bool PAIR>
+__device__ __forceinline__ void load_row(const SysDev& S, bool dia, int row, T (&a)[NE],
+                                         unsigned (&col)[NE])
+{
+    constexpr int KM = (NE - 1) / 2;
+    const int n = S.n;
+#pragma unroll
+    for (int e = 0; e < NE; e++) {
+        a[e] = 0;
+        col[e] = (unsigned)row * sizeof(T);
+    }
+    if (PAIR || dia) {
+        const MatView<T>& M = mv_of<T>(S);
+        const OGSX_GL T* dv = gl(M.dia_val);
+        const OGSX_GL int* off = gl(M.dia_off);
+        const int K = M.dia_k;
+        a[PAIR ? 0 : KM] = dv[row];
+#pragma unroll
+        for (int k = 0; k < KM; k++) {
+            if (k >= K) continue;
+            const int o = off[k], up = min(row + o, n - 1), lo = max(row - o, 0);
+            const OGSX_GL T* u = dv + (int64_t)(k + 1) * n;
+            const int eu = PAIR ? 1 + 2 * k : KM + 1 + k, el = PAIR ? 2 + 2 * k : KM - 1 - k;
+            a[eu] = u[row];
+            col[eu] = (unsigned)up * sizeof(T);
+            a[el] = row - o >= 0 ? u[lo] : (T)0;
+            col[el] = (unsigned)lo * sizeof(T);
+        }
+    } else {
+        const OGSX_GL int* ptr = gl(S.m64.ptr);
+        const OGSX_GL int* cols = gl(S.m64.col);
+        const OGSX_GL double* A = gl(S.A);
+        const int k0 = ptr[row], k1 = ptr[row + 1];
+#pragma unroll
+        for (int e = 0; e < NE; e++)
+            if (k0 + e < k1) {
+                a[e] = (T)A[k0 + e];
+                col[e] = (unsigned)cols[k0 + e] * sizeof(T);
+            }
+    }
+}
+
+template <typename T, int NE, bool PAIR>
+__device__ __forceinline__ T row_sum(const T (&a)[NE], const T (&v)[NE])
+{
+    if constexpr (PAIR) {
+        T s = a[0] * v[0];
+#pragma unroll
+        for (int e = 1; e < NE; e++) s = s + a[e] * v[e];
+        return s;
+    } else {
+#pragma clang fp contract(off)
+        T s = 0;
+#pragma unroll
+        for (int e = 0; e < NE; e++) {
+            const T prod = a[e] * v[e];
+            s = s + prod;
+        }
+        return s;
+    }
+}
+
+template <typename T>
+__device__ __forceinline__ T at_byte(const OGSX_GL T* base, unsigned off)
+{
+    return *(const OGSX_GL T*)((const OGSX_GL char*)base + off);
+}
+
+// A batch of Jacobi-CG iterations (k_cg_spmv, k_cg_update, k_cg_direction)
+// of the members of `g`, one row per thread.  What bounds it: the two
+// exchanges, 1.4-2 us each, and one gather of z.
+template <typename T, int NE, bool PAIR, int VB>
+__global__ __launch_bounds__(kBlock * VB) void k_cg_resident(Grp g, ResLaunch L)
+{
+    // gathers in flight: all of a row's, where the registers allow it
+    constexpr int kBatch = NE * (int)sizeof(T) / 4 * 3 + NE + 28 <= 512 / VB ? NE : (NE + 1) / 2;
+    __shared__ double sw[kSlotVals][4 * VB];
+    __shared__ double sm[kSlotVals][4];
+    __shared__ int flag, ok;
+    const int si = g.blk2sys ? g.blk2sys[blockIdx.x] : 0;
+    const int w = (int)blockIdx.x - (g.blk2sys ? g.blk0[si] : 0);
+    const SysDev& S = g.sys[si];
+    OGSX_GL KrylovState* st = gl(S.st);
+    const bool idle = st->done != 0;
+    const int G = S.G, n = S.n, tid = threadIdx.x;
+    const int it0 = st->iter, max_iter = st->max_iter;
+    const double bnorm = st->bnorm;
+    const double tol = gl(S.prm)->tol, upd_thresh = gl(S.prm)->upd_thresh;
+    double rr = st->rr;
+    ResExchange<VB> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, G / VB,
+                       sw, sm, &ok};
+    if (tid == 0) ok = 1;
+    if (!res_census(L, idle, &flag)) {
+        if (!idle && w == 0 && tid == 0) st->resident = 1;
+        return;
+    }
+    const GVec<T> v = gvec(kv_of<T>(S));
+    // chunk c = w VB + tid / 256, its row tid % 256
+    const int c = w * VB + tid / kBlock, ns = (n + 63) / 64;
+    const int sb = (int)((int64_t)ns * c / G), se = (int)((int64_t)ns * (c + 1) / G);
+    const int mine = sb * 64 + tid % kBlock;
+    const bool have = mine < min(se * 64, n);
+    const int row = have ? mine : n - 1;
+    T a[NE], pj[NE];
+    unsigned col[NE];
+    load_row<T, NE, PAIR>(S, sizeof(T) == 8 && gl(S.prm)->dia, row, a, col);
+    OGSX_GL T* z = wave_uniform(v.s);  // A p stays in registers: its vector carries z
+#pragma unroll
+    for (int e = 0; e < NE; e++) pj[e] = at_byte(v.p, col[e]);
+    T x = v.x[row], r = v.r[row], p = v.p[row];
+    const T d = v.d[row];
+    double error = st->error, alpha_d = st->alpha, rr_old = st->rr_old;
+    int it = it0, done = 0;
+    bool good = true;
+    for (int k = 0; k < L.iters; k++) {
+        const T s = row_sum<T, NE, PAIR>(a, pj);
+        double dot[1] = {have ? (double)p * (double)s : 0.0}, ps[1];
+        good = ex.sum(dot, ps);
+        if (!good) break;
+        alpha_d = rr / ps[0];
+        rr_old = rr;
+        const T alpha = (T)alpha_d;
+        x = x + alpha * p;
+        r = r - alpha * s;
+        const T zi = r / d;
+        if (have) agent_store(z + row, zi);
+        double two[2] = {have ? (double)r * (double)r : 0.0, have ? (double)zi * (double)r : 0.0};
+        double res[2];
+        good = ex.sum(two, res);
+        if (!good) break;
+        const double rnorm = sqrt(res[0]);
+        error = rnorm / bnorm;
+        it++;
+        if (error < tol || rnorm < upd_thresh) {
+            done = error < tol ? 1 : 5;
+            break;
+        }
+        const T beta = (T)(res[1] / rr_old);
+#pragma unroll
+        for (int e0 = 0; e0 < NE; e0 += kBatch) {
+            T zj[kBatch];
+#pragma unroll
+            for (int e = 0; e < kBatch && e0 + e < NE; e++) {
+                // (opaque: keeps one 32-bit offset per entry in registers, not
+                // the 64-bit address the compiler would compute before the loop)
+                asm("" : "+v"(col[e0 + e]));
+                zj[e] = agent_load((const OGSX_GL T*)((const OGSX_GL char*)z + col[e0 + e]));
+            }
+#pragma unroll
+            for (int e = 0; e < kBatch && e0 + e < NE; e++)
+                pj[e0 + e] = zj[e] + beta * pj[e0 + e];
+        }
+        p = zi + beta * p;
+        rr = res[1];
+        if (it >= max_iter) {
+            done = 2;
+            break;
+        }
+    }
+    if (have) {
+        v.x[row] = x;
+        v.r[row] = r;
+        v.p[row] = p;
+    }
+    if (w == 0 && tid == 0) {
+        st->error = error;
+        st->rr = rr;
+        st->rr_old = rr_old;
+        st->alpha = alpha_d;
+        st->iter = it;
+        st->done = done;
+        st->resident = good ? 0 : 2;
+        S.rs->phase = ex.set;
+    }
+}
+
+}  // namespace ogsx
