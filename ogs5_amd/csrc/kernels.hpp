@@ -806,7 +806,9 @@ __device__ __forceinline__ void spmv_crs1(const GMat<VT>& m, const OGSX_GL XT* _
 // SELL-64 or plain CRS format.
 // Symmetric diagonal storage: y_i = d_i x_i + sum_k (u_k[i] x[i + o_k] +
 // u_k[i - o_k] x[i - o_k]), one thread per row, offsets in ascending order
-// and for each the upper, then the lower entry.  Half the matrix values of
+// and for each the upper, then the lower entry, each added by one fused
+// multiply-add (written as such: of a sum of two products the compiler may
+// fuse either, and not the same one in every kernel).  Half the matrix values of
 // the full formats cross HBM; the lower entries are the upper ones of rows
 // o_k back, read again from cache (the blocks of one XCD take consecutive
 // chunks).  Not the reference's summation order: this form serves the FP32
@@ -848,8 +850,8 @@ __device__ __forceinline__ void spmv_symdia_k(const GMat<VT>& m, const OGSX_GL X
                 const int up = min(r[q] + o, n - 1), lo = r[q] - o;
                 const ACC a1 = (ACC)u[r[q]], x1 = (ACC)x[up];  // u[i] = 0 where i + o >= n
                 const ACC a2 = lo >= 0 ? (ACC)u[max(lo, 0)] : (ACC)0, x2 = (ACC)x[max(lo, 0)];
-                s[q] = s[q] + a1 * x1;
-                s[q] = s[q] + a2 * x2;
+                s[q] = fma(a1, x1, s[q]);
+                s[q] = fma(a2, x2, s[q]);
             }
         }
         epi(r[0], s[0]);
@@ -1928,9 +1930,9 @@ __global__ __launch_bounds__(kBlock) void k_cg_init(Grp g, int want)
             const T zi = ri / v.d[i];
             v.r[i] = ri;
             v.p[i] = zi;
-            acc[0] += (double)v.b[i] * (double)v.b[i];
-            acc[1] += (double)ri * (double)ri;
-            acc[2] += (double)ri * (double)zi;
+            acc[0] = fma((double)v.b[i], (double)v.b[i], acc[0]);
+            acc[1] = fma((double)ri, (double)ri, acc[1]);
+            acc[2] = fma((double)ri, (double)zi, acc[2]);
         });
         store_partials<3>(acc, gl(S.part), c.G, b);
     }
@@ -1987,7 +1989,7 @@ __device__ __forceinline__ void cg_spmv_body(const Grp& g, int vb)
         double acc[1] = {0.0};
         spmv_rows<FMT, VT, T, T>(m, v.p, c.G, b, [&](int i, T ax) {
             v.s[i] = ax;
-            acc[0] += (double)v.p[i] * (double)ax;
+            acc[0] = fma((double)v.p[i], (double)ax, acc[0]);
         });
         store_partials<1>(acc, gl(S.part), c.G, b);
     }
@@ -2089,8 +2091,8 @@ __device__ __forceinline__ void cg_update_body(const Grp& g, int vb)
                     const T rn = ri[u] - alpha * si[u];
                     store_hint<VNT>(r + k, rn);
                     const T zi = rn / di[u];
-                    acc[0] += (double)rn * (double)rn;
-                    acc[1] += (double)zi * (double)rn;
+                    acc[0] = fma((double)rn, (double)rn, acc[0]);
+                    acc[1] = fma((double)zi, (double)rn, acc[1]);
                 }
             }
             i = end;
@@ -2114,8 +2116,8 @@ __device__ __forceinline__ void cg_update_body(const Grp& g, int vb)
                 const T rn = ri[u] - alpha * si[u];
                 store_hint<VNT>(r + k, rn);
                 const T zi = rn / di[u];
-                acc[0] += (double)rn * (double)rn;
-                acc[1] += (double)zi * (double)rn;
+                acc[0] = fma((double)rn, (double)rn, acc[0]);
+                acc[1] = fma((double)zi, (double)rn, acc[1]);
             }
         }
         if (tail) {  // the batch loop ran once: i is the thread's extra row
@@ -2123,8 +2125,8 @@ __device__ __forceinline__ void cg_update_body(const Grp& g, int vb)
             const T rn = rt - alpha * st1;
             store_hint<VNT>(r + i, rn);
             const T zi = rn / dt;
-            acc[0] += (double)rn * (double)rn;
-            acc[1] += (double)zi * (double)rn;
+            acc[0] = fma((double)rn, (double)rn, acc[0]);
+            acc[1] = fma((double)zi, (double)rn, acc[1]);
             i = end;
         }
         for (; i < end; i += kBlock) {
@@ -2132,8 +2134,8 @@ __device__ __forceinline__ void cg_update_body(const Grp& g, int vb)
             const T rn = r[i] - alpha * sv[i];
             r[i] = rn;
             const T zi = rn / d[i];
-            acc[0] += (double)rn * (double)rn;
-            acc[1] += (double)zi * (double)rn;
+            acc[0] = fma((double)rn, (double)rn, acc[0]);
+            acc[1] = fma((double)zi, (double)rn, acc[1]);
         }
         store_partials<2>(acc, gl(S.part) + 4 * part_stride(c.G), c.G, b);
     }
@@ -2268,8 +2270,8 @@ __global__ __launch_bounds__(kBlock) void k_cg_rescan(Grp g)
         vec_chunk(S.n, c.G, b, [&](int i) {
             const T ri = v.r[i];
             const T zi = ri / v.d[i];
-            acc[0] += (double)ri * (double)ri;
-            acc[1] += (double)zi * (double)ri;
+            acc[0] = fma((double)ri, (double)ri, acc[0]);
+            acc[1] = fma((double)zi, (double)ri, acc[1]);
         });
         store_partials<2>(acc, gl(S.part) + 4 * part_stride(c.G), c.G, b);
     }
@@ -2317,9 +2319,9 @@ __global__ __launch_bounds__(kBlock) void k_bi_init(Grp g, int want)
             v.r[i] = ri;
             v.v[i] = 0;
             v.p[i] = 0;
-            acc[0] += (double)ri * (double)ri;
-            acc[1] += (double)ri * (double)ri;
-            acc[2] += (double)v.b[i] * (double)v.b[i];
+            acc[0] = fma((double)ri, (double)ri, acc[0]);
+            acc[1] = fma((double)ri, (double)ri, acc[1]);
+            acc[2] = fma((double)v.b[i], (double)v.b[i], acc[2]);
         });
         store_partials<3>(acc, gl(S.part), c.G, b);
     }
@@ -2450,7 +2452,7 @@ __device__ __forceinline__ void bi_spmv_v_body(const Grp& g, int vb)
         double acc[1] = {0.0};
         spmv_rows<FMT, VT, T, T>(m, v.ph, c.G, b, [&](int i, T ax) {
             v.v[i] = ax;
-            acc[0] += (double)v.r0[i] * (double)ax;
+            acc[0] = fma((double)v.r0[i], (double)ax, acc[0]);
         });
         store_partials<1>(acc, gl(S.part) + 4 * part_stride(c.G), c.G, b);
     }
@@ -2499,7 +2501,7 @@ __device__ __forceinline__ void bi_s_body(const Grp& g, int vb)
                 const T si = rr[u] - alpha * vv[u];
                 v.s[k] = si;
                 v.sh[k] = si / dd[u];
-                acc[0] += (double)si * (double)si;
+                acc[0] = fma((double)si, (double)si, acc[0]);
             });
         store_partials<1>(acc, gl(S.part) + 8 * part_stride(c.G), c.G, b);
     }
@@ -2543,8 +2545,8 @@ __device__ __forceinline__ void bi_spmv_t_body(const Grp& g, int vb)
         double acc[2] = {0.0, 0.0};
         spmv_rows<FMT, VT, T, T>(m, v.sh, c.G, b, [&](int i, T ax) {
             v.t[i] = ax;
-            acc[0] += (double)ax * (double)ax;
-            acc[1] += (double)ax * (double)v.s[i];
+            acc[0] = fma((double)ax, (double)ax, acc[0]);
+            acc[1] = fma((double)ax, (double)v.s[i], acc[1]);
         });
         store_partials<2>(acc, gl(S.part) + 12 * part_stride(c.G), c.G, b);
     }
@@ -2596,8 +2598,8 @@ __device__ __forceinline__ void bi_update_body(const Grp& g, int vb)
                 v.x[k] = xx[u] + (alpha * ph[u] + omega * sh[u]);
                 const T ri = ss[u] - omega * tt[u];
                 v.r[k] = ri;
-                acc[0] += (double)ri * (double)ri;
-                acc[1] += (double)r0[u] * (double)ri;
+                acc[0] = fma((double)ri, (double)ri, acc[0]);
+                acc[1] = fma((double)r0[u], (double)ri, acc[1]);
             });
         store_partials<2>(acc, gl(S.part), c.G, b);
     }
@@ -2760,10 +2762,10 @@ __global__ __launch_bounds__(kBlock) void k_ir_residual(Grp g)
         spmv_rows<FMT, double, double, double>(m, v.x, c.G, b, [&](int i, double ax) {
             const double ri = v.b[i] - ax;
             r[i] = ri;
-            acc[0] += v.b[i] * v.b[i];
-            acc[1] += ri * ri;
+            acc[0] = fma(v.b[i], v.b[i], acc[0]);
+            acc[1] = fma(ri, ri, acc[1]);
             const double si = scaled ? (double)sc[i] * ri : ri;
-            acc[2] += si * si;
+            acc[2] = fma(si, si, acc[2]);
         });
         store_partials<3>(acc, gl(S.part), c.G, b);
     }
@@ -2996,9 +2998,9 @@ __global__ __launch_bounds__(kBlock) void k_cg1_init(Grp g, int want)
     spmv_rows<FMT, VT, T, T>(m, v.x, c.G, c.b, [&](int i, T ax) {
         const T ri = v.b[i] - ax;
         v.r[i] = ri;
-        acc[0] += (double)v.b[i] * (double)v.b[i];
-        acc[1] += (double)ri * (double)ri;
-        acc[2] += (double)ri * (double)ri;
+        acc[0] = fma((double)v.b[i], (double)v.b[i], acc[0]);
+        acc[1] = fma((double)ri, (double)ri, acc[1]);
+        acc[2] = fma((double)ri, (double)ri, acc[2]);
     });
     store_partials<3>(acc, gl(S.part), c.G, c.b);
 }
@@ -3019,8 +3021,8 @@ __device__ __forceinline__ void cg1_spmv_body(const Grp& g, int resume, int vb)
     spmv_rows<FMT, VT, T, T>(m, v.r, c.G, c.b, [&](int i, T ax) {
         v.z[i] = ax;
         const T ri = v.r[i];
-        acc[0] += (double)ri * (double)ax;
-        acc[1] += (double)ri * (double)ri;
+        acc[0] = fma((double)ri, (double)ax, acc[0]);
+        acc[1] = fma((double)ri, (double)ri, acc[1]);
     });
     store_partials<2>(acc, gl(S.part), c.G, c.b);
     if (c.b == 0 && threadIdx.x == 0) {
@@ -3171,7 +3173,7 @@ __global__ __launch_bounds__(kBlock) void k_cg1_resume(Grp g)
         const T sn = v.z[i] + beta * v.s[i];
         v.p[i] = pn;
         v.s[i] = sn;
-        acc[0] += (double)pn * (double)sn;
+        acc[0] = fma((double)pn, (double)sn, acc[0]);
     });
     store_partials<1>(acc, gl(S.part) + 4 * part_stride(c.G), c.G, c.b);
     if (c.b == 0 && threadIdx.x == 0) st->rr = gamma;

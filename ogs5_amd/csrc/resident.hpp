@@ -285,7 +285,7 @@ __device__ __forceinline__ T row_sum(const T (&a)[NE], const T (&v)[NE])
     if constexpr (PAIR) {
         T s = a[0] * v[0];
 #pragma unroll
-        for (int e = 1; e < NE; e++) s = s + a[e] * v[e];
+        for (int e = 1; e < NE; e++) s = fma(a[e], v[e], s);
         return s;
     } else {
 #pragma clang fp contract(off)
