@@ -16,6 +16,7 @@
 #include <string>
 #include <map>
 #include <thread>
+#include <tuple>
 #include <vector>
 
 #include "kernels.hpp"
@@ -43,18 +44,14 @@ int fail(int code, const std::string& msg)
 // Blocks of the n-sized kernels of one system (each block a contiguous chunk
 // of rows).  G sets the partial-sum layout, so it is a function of n alone,
 // never tuned at run time: one row per thread up to kResMaxRows rows (the
-// systems that resident launches hold on the chip, a thread per row), then
-// OGSX_ROWS_PER_BLOCK rows per block, at most kMaxGrid (2048) blocks (the
-// partial sums' reduction loads all of them in one batch).  Many rows per
-// block cut block dispatches and the per-block reduction of partial sums.
-#ifndef OGSX_ROWS_PER_BLOCK
-#define OGSX_ROWS_PER_BLOCK 1024
-#endif
-
+// systems that resident launches hold on the chip, a thread per row); 1024
+// blocks, four to a compute unit, for the sizes whose vectors fit the chip's
+// LDS; then kMaxGrid (2048) blocks (the partial sums' reduction loads all of
+// them in one batch).
 int grid_for(int64_t n)
 {
     int64_t g = n <= kResMaxRows ? (n + kBlock - 1) / kBlock
-                                 : (n + OGSX_ROWS_PER_BLOCK - 1) / OGSX_ROWS_PER_BLOCK;
+                                 : n <= kStreamMaxRows ? kStreamBlocks : kMaxGrid;
     g = (g + kNumXcd - 1) / kNumXcd * kNumXcd;
     return (int)std::max<int64_t>(kNumXcd, std::min<int64_t>(g, kMaxGrid));
 }

@@ -62,10 +62,43 @@ __device__ __forceinline__ void row_chunk(int n, int G, int b, int& beg, int& en
     end = min(se * 64, n);
 }
 
+// Thread of the 256 that share a chunk (a workgroup of the resident kernels
+// has several chunks).
+__device__ __forceinline__ int chunk_thread() { return (int)threadIdx.x % kBlock; }
+
+// v of lane l + OFF in lane l, for the lanes the sum below reads (OFF = 32 and
+// 16: the halves of the wave and the rows of 16 change places; below: a DPP
+// row shift).
+template <int OFF>
+__device__ __forceinline__ int lanes_down(int v)
+{
+    if constexpr (OFF == 32)
+        return (int)__builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false)[1];
+    else if constexpr (OFF == 16)
+        return (int)__builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false)[1];
+    else
+        return __builtin_amdgcn_update_dpp(0, v, 0x100 + OFF, 0xf, 0xf, true);
+}
+template <int OFF>
+__device__ __forceinline__ double lanes_down(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = (unsigned)lanes_down<OFF>((int)b);
+    const unsigned hi = (unsigned)lanes_down<OFF>((int)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// Sum over the wave, in lane 0: v[l] + v[l + 32], then 16, 8, 4, 2, 1.  By
+// lane swaps and DPP shifts, not through LDS (__shfl_down): the sums are on
+// the serial path of every dot product.
 __device__ __forceinline__ double wave_sum(double v)
 {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+    v += lanes_down<32>(v);
+    v += lanes_down<16>(v);
+    v += lanes_down<8>(v);
+    v += lanes_down<4>(v);
+    v += lanes_down<2>(v);
+    v += lanes_down<1>(v);
     return v;
 }
 
@@ -794,7 +827,7 @@ __device__ __forceinline__ void spmv_crs1(const GMat<VT>& m, const OGSX_GL XT* _
 #pragma clang fp contract(off)
     int beg, end;
     row_chunk(m.n, G, b, beg, end);
-    for (int r = beg + (int)threadIdx.x; r < end; r += kBlock) {
+    for (int r = beg + chunk_thread(); r < end; r += kBlock) {
         const int k1 = m.ptr[r + 1];
         ACC s = 0;
         for (int k = m.ptr[r]; k < k1; k++) s += (ACC)m.val[k] * (ACC)x[m.col[k]];
@@ -833,7 +866,7 @@ __device__ __forceinline__ void spmv_symdia_k(const GMat<VT>& m, const OGSX_GL X
     // 4 gave 36.1, 35.5, 43.8 us before the offset loop was unrolled; unrolled
     // R = 1, 2: 31.5, 31.4 us)
     constexpr int R = OGSX_DIA_ROWS;
-    for (int i = beg + threadIdx.x; i < end; i += R * kBlock) {
+    for (int i = beg + chunk_thread(); i < end; i += R * kBlock) {
         int r[R];
 #pragma unroll
         for (int q = 0; q < R; q++) r[q] = min(i + q * kBlock, end - 1);
@@ -886,7 +919,7 @@ __device__ __forceinline__ void spmv_symdia_crs_k(const GMat<VT>& m, const OGSX_
     // (72 VGPRs, 7 waves)
     constexpr int R = 1;
     constexpr int kUnroll = KC > 0 ? KC : 4;
-    for (int i = beg + threadIdx.x; i < end; i += R * kBlock) {
+    for (int i = beg + chunk_thread(); i < end; i += R * kBlock) {
         int r[R];
 #pragma unroll
         for (int q = 0; q < R; q++) r[q] = min(i + q * kBlock, end - 1);

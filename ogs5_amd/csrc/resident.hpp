@@ -46,6 +46,12 @@ constexpr int kSlotVals = 3;    // values of one exchange
 constexpr int kSlotCopies = 8;
 constexpr int kResMaxSlots = kBlock;          // slots per value and copy
 constexpr int kResMaxRows = 1 << 18;          // rows of a resident system
+// Larger systems whose vectors fit the LDS of 256 workgroups (k_cg_stream):
+// 1024 chunks, four to a workgroup, of up to 9 rows per thread.
+constexpr int kStreamVb = 4;
+constexpr int kStreamBlocks = 1024;
+constexpr int kStreamSlots = 9;
+constexpr int kStreamMaxRows = kStreamBlocks * kStreamSlots * kBlock;
 constexpr unsigned kResPolls = 1u << 21;      // polls of one wait (seconds)
 constexpr long long kCensusTicks = 20000;     // 100 MHz: 200 us
 constexpr int kCensusRing = 64;
@@ -172,29 +178,56 @@ struct ResExchange {
         return slot + ((size_t)(s * kSlotVals + k) * kSlotCopies + copy) * slots;
     }
 
+    // Waits for every workgroup of the system (an exchange of nothing):
+    // vector entries published before it can be read after it.
+    template <typename F>
+    __device__ __forceinline__ bool barrier(F&& meanwhile)
+    {
+        const double none[1] = {0.0};
+        double out[1];
+        return sum<1, false>(none, out, meanwhile);
+    }
+
     template <int NV>
     __device__ __forceinline__ bool sum(const double (&v)[NV], double (&out)[NV])
     {
+        return sum<NV, true>(v, out, [] {});
+    }
+
+    // meanwhile(): loads to issue once this workgroup has posted its sums
+    template <int NV, bool VALUES, typename F>
+    __device__ __forceinline__ bool sum(const double (&v)[NV], double (&out)[NV], F&& meanwhile)
+    {
         const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
         const int per = VB / q;  // slots this workgroup posts per value
+        if constexpr (VALUES) {
 #pragma unroll
-        for (int k = 0; k < NV; k++) {
-            const double s = wave_sum(v[k]);
-            if (lane == 0) sw[k][wave] = s;
+            for (int k = 0; k < NV; k++) {
+                const double s = wave_sum(v[k]);
+                if (lane == 0) sw[k][wave] = s;
+            }
         }
         wait_memory();  // vector entries published before this exchange
         __syncthreads();
         const int copy = t % kSlotCopies, j = t / kSlotCopies % per, kk = t / kSlotCopies / per;
         if (kk < NV) {
             double s = 0.0;
-            for (int i = 0; i < q; i++) {
-                const double* c = &sw[kk][4 * (j * q + i)];
-                s += ((c[0] + c[1]) + c[2]) + c[3];
+            if constexpr (VALUES) {
+                // (all of the sums read before the first is added)
+                double c[VB][4];
+#pragma unroll
+                for (int i = 0; i < VB; i++)
+#pragma unroll
+                    for (int x = 0; x < 4; x++) c[i][x] = sw[kk][4 * min(j * q + i, VB - 1) + x];
+#pragma unroll
+                for (int i = 0; i < VB; i++)
+                    if (i < q) s += ((c[i][0] + c[i][1]) + c[i][2]) + c[i][3];
             }
             unsigned long long bits = (unsigned long long)__double_as_longlong(s);
             if (bits == kSlotEmpty) bits = 0x7FF8000000000000ull;
             agent_store(at(set, kk, copy) + w * per + j, bits);
         }
+        meanwhile();
         if (wave < 4) {
             unsigned long long got[NV];
 #pragma unroll
@@ -214,15 +247,19 @@ struct ResExchange {
                     }
                 }
             }
+            if constexpr (VALUES) {
 #pragma unroll
-            for (int k = 0; k < NV; k++) {
-                const double s = wave_sum(__longlong_as_double((long long)got[k]));
-                if (lane == 0) sm[k][wave] = s;
+                for (int k = 0; k < NV; k++) {
+                    const double s = wave_sum(__longlong_as_double((long long)got[k]));
+                    if (lane == 0) sm[k][wave] = s;
+                }
             }
         }
         __syncthreads();
+        if constexpr (VALUES) {
 #pragma unroll
-        for (int k = 0; k < NV; k++) out[k] = ((sm[k][0] + sm[k][1]) + sm[k][2]) + sm[k][3];
+            for (int k = 0; k < NV; k++) out[k] = ((sm[k][0] + sm[k][1]) + sm[k][2]) + sm[k][3];
+        }
         // every workgroup has read the previous set: empty this one's slots
         // there (it is used again two exchanges on)
         const int prev = set == 0 ? kSlotSets - 1 : set - 1;
@@ -412,5 +449,336 @@ __global__ __launch_bounds__(kBlock * VB) void k_cg_resident(Grp g, ResLaunch L)
         S.rs->phase = ex.set;
     }
 }
+
+// The symmetric diagonal copy as k_cg_stream reads it: KC offsets and every
+// array's base in scalar registers.
+template <int KC, typename T>
+struct DiaRows {
+    const OGSX_GL T* dv;
+    int off[KC];
+    int n;
+
+    __device__ __forceinline__ explicit DiaRows(const MatView<T>& m)
+    {
+        dv = wave_uniform(gl(const_cast<T*>(m.dia_val)));
+        n = __builtin_amdgcn_readfirstlane(m.n);
+#pragma unroll
+        for (int k = 0; k < KC; k++) off[k] = __builtin_amdgcn_readfirstlane(gl(m.dia_off)[k]);
+    }
+
+    // The products' factors of entries e0 .. e1 of row r: matrix value and x.
+    // Entries are in CRS column order: KC - 1 - k the lower entry of offset k,
+    // KC the diagonal, KC + 1 + k the upper.  EDGE: the row may reach past the
+    // first or last one (indices clamped, such a value taken as 0).
+    template <bool EDGE, int E0, int E1, bool A = true, bool X = true>
+    __device__ __forceinline__ void load(const OGSX_GL T* x, int r, T* a, T* xv) const
+    {
+        const unsigned sz = sizeof(T), at = (unsigned)r * sz;
+#pragma unroll
+        for (int e = E0; e < E1; e++) {
+            const int k = e < KC ? KC - 1 - e : e > KC ? e - KC - 1 : 0;
+            const int o = e < KC ? -off[k] : e > KC ? off[k] : 0;
+            const unsigned dia = e == KC ? 0u : (unsigned)((k + 1) * n);  // its array
+            if constexpr (EDGE) {
+                const int j = min(max(r + o, 0), n - 1);
+                if constexpr (A) a[e - E0] = at_byte(dv, sz * (dia + (unsigned)(e < KC ? j : r)));
+                if constexpr (X) xv[e - E0] = at_byte(x, sz * (unsigned)j);
+            } else {
+                // 32-bit offsets from two bases: (KC + 1) n values are under 4 GB
+                if constexpr (A) a[e - E0] = at_byte(dv, at + sz * (dia + (unsigned)(e < KC ? o : 0)));
+                if constexpr (X) xv[e - E0] = at_byte(x, at + sz * (unsigned)o);
+            }
+        }
+    }
+
+    // The loads above are issued before anything below uses one (left alone,
+    // the compiler takes the row two loads and one round trip at a time).
+    static __device__ __forceinline__ void issued() { asm volatile("" ::: "memory"); }
+
+    // Matrix values of the entries a row sum takes first (FP32 all of them).
+    static constexpr int kFirst = sizeof(T) == 4 ? 2 * KC + 1 : KC;
+    __device__ __forceinline__ bool inner(int r) const
+    {
+        // the wave's 64 rows are consecutive: one test for all of them
+        const int lead = __builtin_amdgcn_readfirstlane(r);
+        return lead - off[KC - 1] >= 0 && lead + 63 + off[KC - 1] < n;
+    }
+    __device__ __forceinline__ void prefetch(int r, T* a) const
+    {
+        if (inner(r))
+            load<false, 0, kFirst, true, false>(nullptr, r, a, nullptr);
+        else
+            load<true, 0, kFirst, true, false>(nullptr, r, a, nullptr);
+    }
+
+    // Lower entries of a row that reaches past the first one are 0 (upper
+    // ones past the last are stored so).
+    template <bool EDGE>
+    __device__ __forceinline__ void mask(int r, T* a) const
+    {
+        if constexpr (EDGE) {
+#pragma unroll
+            for (int e = 0; e < KC; e++) a[e] = r >= off[KC - 1 - e] ? a[e] : (T)0;
+        }
+    }
+
+    // Row sum of row r in the order of spmv_symdia_k (FP32) or
+    // spmv_symdia_crs_k (FP64).  FP32 takes the row's 2 x 27 loads at once,
+    // FP64 (twice the registers) its lower and its upper half.
+    // PRE: its first values are in `a` already.
+    template <bool EDGE, bool PRE>
+    __device__ __forceinline__ T sum(const OGSX_GL T* x, int r, T* a) const
+    {
+        constexpr int NE = 2 * KC + 1;
+        if constexpr (sizeof(T) == 4) {
+            T xv[NE];
+            load<EDGE, 0, NE, !PRE>(x, r, a, xv);
+            issued();
+            mask<EDGE>(r, a);
+            T s = a[KC] * xv[KC];
+#pragma unroll
+            for (int k = 0; k < KC; k++) {
+                s = fma(a[KC + 1 + k], xv[KC + 1 + k], s);
+                s = fma(a[KC - 1 - k], xv[KC - 1 - k], s);
+            }
+            return s;
+        } else {
+#pragma clang fp contract(off)
+            T xv[KC], a2[KC + 1], xv2[KC + 1];
+            load<EDGE, 0, KC, !PRE>(x, r, a, xv);
+            issued();
+            mask<EDGE>(r, a);
+            T s = 0;
+#pragma unroll
+            for (int e = 0; e < KC; e++) {
+                const T prod = a[e] * xv[e];
+                s = s + prod;
+            }
+            load<EDGE, KC, NE>(x, r, a2, xv2);
+            issued();
+#pragma unroll
+            for (int e = 0; e <= KC; e++) {
+                const T prod = a2[e] * xv2[e];
+                s = s + prod;
+            }
+            return s;
+        }
+    }
+
+    // epi(row, sum) of the thread's rows r, r + 256, ... < end; pre holds the
+    // first row's first values.
+    template <typename Epi>
+    __device__ __forceinline__ void rows(const OGSX_GL T* x, int r, int end, const T (&pre)[kFirst],
+                                         Epi&& epi) const
+    {
+        if (r >= end) return;
+        asm("" : "+v"(r));
+        T a[kFirst];
+#pragma unroll
+        for (int e = 0; e < kFirst; e++) a[e] = pre[e];
+        epi(r, inner(r) ? sum<false, true>(x, r, a) : sum<true, true>(x, r, a));
+#pragma nounroll
+        for (r += kBlock; r < end; r += kBlock) {
+            asm("" : "+v"(r));  // opaque: no induction variable, hence register, per load
+            T b[kFirst];
+            epi(r, inner(r) ? sum<false, false>(x, r, b) : sum<true, false>(x, r, b));
+        }
+    }
+};
+
+// A batch of Jacobi-CG iterations of one system too large for a thread per
+// row: 256 workgroups hold its vectors in LDS (a thread's rows are those of
+// the separate launches, up to 9) and stream the symmetric diagonal copy of
+// the matrix (KC offsets) from memory.  p is gathered through the caches: it is published into one of
+// four vectors in turn, and once in four iterations one wave per workgroup
+// invalidates its compute unit's and XCD's caches (0.25 us an iteration; every
+// iteration 1.6 us, by every wave 28 us), so that no gather finds a line of
+// that vector's previous use.  Three exchanges per iteration: (p, s), then
+// (r, r) and (z, r), then the new p.
+//
+// Per iteration on 128^3 hexes (FP32): 39 us, 61 with three launches (the
+// time is the matrix, 23 us, then the exchanges); on 85 x 64 x 53 (FP64) 19
+// and 31 us (the latency of two rows of loads and of the exchanges).
+//
+// XL, PL: x and p in LDS too; without, x stays in memory (read and written
+// by its row's thread alone) and a row's own p is read back from where it was
+// published.  LDS sets which: 160 KB hold 9 rows per thread of four FP32
+// vectors, or 4, 6 or 9 of four, three or two FP64 ones.
+template <int KC, typename T, bool XL, bool PL>
+__global__ __launch_bounds__(kBlock * kStreamVb) void k_cg_stream(Grp g, ResLaunch L)
+{
+    constexpr int VB = kStreamVb, NT = kBlock * VB;
+    extern __shared__ __align__(16) char stream_lds[];
+    __shared__ double sw[kSlotVals][4 * VB];
+    __shared__ double sm[kSlotVals][4];
+    __shared__ int flag, ok;
+    const int si = g.blk2sys ? g.blk2sys[blockIdx.x] : 0;
+    const int launched = (int)blockIdx.x - (g.blk2sys ? g.blk0[si] : 0);
+    const SysDev& S = g.sys[si];
+    OGSX_GL KrylovState* st = gl(S.st);
+    const bool idle = st->done != 0;
+    const int G = S.G, n = S.n, tid = threadIdx.x, nwg = G / VB;
+    // workgroups are dealt to the XCDs in turn: each XCD gets neighbouring chunks
+    const int w = nwg % kNumXcd ? launched
+                                : (launched % kNumXcd) * (nwg / kNumXcd) + launched / kNumXcd;
+    const int it0 = st->iter, max_iter = st->max_iter;
+    const double bnorm = st->bnorm;
+    const double tol = gl(S.prm)->tol, upd_thresh = gl(S.prm)->upd_thresh;
+    double rr = st->rr;
+    ResExchange<VB> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, nwg, sw, sm, &ok};
+    if (tid == 0) ok = 1;
+    if (!res_census(L, idle, &flag)) {
+        if (!idle && w == 0 && tid == 0) st->resident = 1;
+        return;
+    }
+    const DiaRows<KC, T> m(mv_of<T>(S));
+    const GVec<T> v = gvec(kv_of<T>(S));
+    OGSX_GL T* const vd = wave_uniform(v.d);
+    OGSX_GL T* const vx = wave_uniform(v.x);
+    const int c = w * VB + tid / kBlock, ns = (n + 63) / 64;
+    const int beg = (int)((int64_t)ns * c / G) * 64;
+    const int end = min((int)((int64_t)ns * (c + 1) / G) * 64, n);
+    const int first = beg + chunk_thread();
+    // row first + 256 j lives at [1024 j + tid] of each vector in LDS
+    const int stride = ((ns + G - 1) / G * 64 + kBlock - 1) / kBlock * NT;
+    T* const rl = (T*)stream_lds + tid;
+    T* const sl = rl + stride;
+    T* const pl = sl + stride;
+    T* const xl = pl + stride;
+    auto at = [&](int row) { return (row - first) * VB; };
+    for (int i = first; i < end; i += kBlock) {
+        rl[at(i)] = v.r[i];
+        if constexpr (PL) pl[at(i)] = v.p[i];
+        if constexpr (XL) xl[at(i)] = v.x[i];
+    }
+    // (CG leaves these vectors unused)
+    OGSX_GL T* const ring[4] = {wave_uniform(v.r0), wave_uniform(v.v), wave_uniform(v.t),
+                                wave_uniform(v.ph)};
+    const OGSX_GL T* src = wave_uniform(v.p);
+    // the first row's first matrix values, loaded while the exchange before
+    // their use waits; likewise the rows' diagonal entries
+    T pre[DiaRows<KC, T>::kFirst];
+    // (opaque row numbers: nothing of a row is computed ahead of the loop and
+    // kept in registers)
+    auto ahead = [&] {
+        int i = min(first, end - 1);
+        asm("" : "+v"(i));
+        m.prefetch(i, pre);
+    };
+    T dj[kStreamSlots];
+    auto diagonal = [&] {
+        int i = first;
+        asm("" : "+v"(i));
+#pragma unroll
+        for (int j = 0; j < kStreamSlots; j++) dj[j] = 1;
+#pragma unroll
+        for (int j = 0; j < kStreamSlots; j++)
+            if (i + j * kBlock < end) dj[j] = at_byte(vd, (unsigned)(i + j * kBlock) * sizeof(T));
+    };
+    ahead();
+    double error = st->error, alpha_d = st->alpha, rr_old = st->rr_old;
+    int it = it0, done = 0;
+    bool good = true;
+    for (int k = 0; k < L.iters; k++) {
+        double dot[1] = {0.0}, ps[1];
+        m.rows(src, first, end, pre, [&](int row, T ax) {
+            T pi;
+            if constexpr (PL)
+                pi = pl[at(row)];
+            else
+                pi = src[row];
+            sl[at(row)] = ax;
+            dot[0] = fma((double)pi, (double)ax, dot[0]);
+        });
+        good = ex.template sum<1, true>(dot, ps, diagonal);
+        if (!good) break;
+        alpha_d = rr / ps[0];
+        rr_old = rr;
+        const T alpha = (T)alpha_d;
+        double two[2] = {0.0, 0.0}, res[2];
+        int start = first;
+        asm("" : "+v"(start));
+#pragma unroll
+        for (int j = 0; j < kStreamSlots; j++) {
+            const int i = start + j * kBlock;
+            if (i >= end) break;
+            T pi;
+            if constexpr (PL)
+                pi = pl[at(i)];
+            else
+                pi = src[i];
+            if constexpr (XL)
+                xl[at(i)] = xl[at(i)] + alpha * pi;
+            else
+                vx[i] = vx[i] + alpha * pi;
+            const T rn = rl[at(i)] - alpha * sl[at(i)];
+            rl[at(i)] = rn;
+            const T zi = rn / dj[j];
+            sl[at(i)] = zi;  // A p is done with
+            two[0] = fma((double)rn, (double)rn, two[0]);
+            two[1] = fma((double)zi, (double)rn, two[1]);
+        }
+        good = ex.sum(two, res);
+        if (!good) break;
+        const double rnorm = sqrt(res[0]);
+        error = rnorm / bnorm;
+        it++;
+        if (error < tol || rnorm < upd_thresh) {
+            done = error < tol ? 1 : 5;
+            break;
+        }
+        const T beta = (T)(res[1] / rr_old);
+        OGSX_GL T* to = k & 2 ? (k & 1 ? ring[3] : ring[2]) : (k & 1 ? ring[1] : ring[0]);
+        for (int i = first; i < end; i += kBlock) {
+            T pi;
+            if constexpr (PL)
+                pi = pl[at(i)];
+            else
+                pi = src[i];
+            pi = sl[at(i)] + beta * pi;
+            if constexpr (PL) pl[at(i)] = pi;
+            agent_store(to + i, pi);
+        }
+        src = to;
+        rr = res[1];
+        if (it >= max_iter) {
+            done = 2;
+            break;
+        }
+        good = ex.barrier(ahead);
+        if (!good) break;
+        if ((k & 3) == 0) {
+            if (tid < 64) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            __syncthreads();
+        }
+    }
+    const GVec<T> out = gvec(kv_of<T>(S));
+    for (int i = first; i < end; i += kBlock) {
+        out.r[i] = rl[at(i)];
+        if constexpr (PL)
+            out.p[i] = pl[at(i)];
+        else
+            out.p[i] = agent_load(src + i);
+        if constexpr (XL) out.x[i] = xl[at(i)];
+    }
+    if (w == 0 && tid == 0) {
+        st->error = error;
+        st->rr = rr;
+        st->rr_old = rr_old;
+        st->alpha = alpha_d;
+        st->iter = it;
+        st->done = done;
+        st->resident = good ? 0 : 2;
+        S.rs->phase = ex.set;
+    }
+}
+
+// Bytes of LDS that one vector of k_cg_stream takes.
+constexpr size_t stream_vec_bytes(int n, int G, size_t size)
+{
+    const int ns = (n + 63) / 64;
+    return (size_t)(((ns + G - 1) / G * 64 + kBlock - 1) / kBlock) * kBlock * kStreamVb * size;
+}
+constexpr size_t kStreamLds = 160 * 1024 - 1024;  // a compute unit's, less the exchange's
 
 }  // namespace ogsx
