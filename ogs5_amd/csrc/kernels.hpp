@@ -2334,6 +2334,22 @@ __global__ __launch_bounds__(kBlock) void k_cg_resume(Grp g)
 // Partial layout: [0,2G) (r,r),(r0,r); [4G,5G) (r0,v); [8G,9G) (s,s);
 // [12G,14G) (t,t),(t,s).
 
+// Its updates of p and x, each operation written out: of sums of products the
+// compiler may fuse one or another, and not the same in every kernel.
+template <typename T>
+__device__ __forceinline__ T bi_p(T r, T beta, T p, T omega, T v)
+{
+#pragma clang fp contract(off)
+    return fma(beta, fma(-omega, v, p), r);
+}
+template <typename T>
+__device__ __forceinline__ T bi_x(T x, T alpha, T ph, T omega, T sh)
+{
+#pragma clang fp contract(off)
+    const T step = fma(alpha, ph, omega * sh);
+    return x + step;
+}
+
 // s = A x; r0 = b - s; r = r0; v = p = 0; partials (r,r), (r0,r), (b,b)
 template <int FMT, typename VT, typename T>
 __global__ __launch_bounds__(kBlock) void k_bi_init(Grp g, int want)
@@ -2457,7 +2473,7 @@ __device__ __forceinline__ void bi_dir_body(const Grp& g, int vb)
             return true;
         },
         [&](int k, int u) {
-            const T pi = it == 0 ? rr[u] : rr[u] + beta * (pp[u] - omega * vv[u]);
+            const T pi = it == 0 ? rr[u] : bi_p(rr[u], beta, pp[u], omega, vv[u]);
             v.p[k] = pi;
             v.ph[k] = pi / dd[u];
         });
@@ -2628,7 +2644,7 @@ __device__ __forceinline__ void bi_update_body(const Grp& g, int vb)
                 return true;
             },
             [&](int k, int u) {
-                v.x[k] = xx[u] + (alpha * ph[u] + omega * sh[u]);
+                v.x[k] = bi_x(xx[u], alpha, ph[u], omega, sh[u]);
                 const T ri = ss[u] - omega * tt[u];
                 v.r[k] = ri;
                 acc[0] = fma((double)ri, (double)ri, acc[0]);

@@ -82,6 +82,29 @@ def test_cg_rows_read_from_crs(kind, shape, prec):
         system[1].close()
 
 
+# sizes as above; the largest resident system of 256-thread workgroups
+# (65,536 rows) and of 512-thread ones (131,072) and the next one up
+BI = [("line", (1,)), ("line", (255,)), ("line", (2048,)), ("quad", (1, 1)), ("quad", (33, 21)),
+      ("quad", (361, 361)), ("quad", (361, 362)), ("tet", (1, 1, 1)), ("tet", (9, 7, 5)),
+      ("tet", (39, 39, 39)), ("tet", (40, 40, 40)), ("tet", (50, 50, 50)),
+      ("hex", (1, 1, 1)), ("hex", (9, 7, 5)), ("hex", (39, 39, 39)), ("hex", (40, 40, 40))]
+
+
+@pytest.mark.parametrize("prec", [ox.FP64, ox.FP32_IR])
+@pytest.mark.parametrize("kind,shape", BI)
+def test_bicgstab_equals_separate_launches(kind, shape, prec):
+    """Row-only elimination (rows read from CRS) and the symmetric one (from
+    the diagonal copy); stops at a limit and at the tolerance."""
+    sc = _scenario(kind, shape)
+    system = W.make_system(sc, prec)
+    for bc in (ox.DIRICHLET_ROW, ox.DIRICHLET_SYMMETRIC):
+        for max_iter in (1, 30):
+            sc.max_iter = max_iter
+            kw = dict(method=ox.BICGSTAB, dirichlet=bc)
+            _same(_solve(sc, system, False, **kw), _solve(sc, system, True, **kw))
+    system[1].close()
+
+
 @pytest.mark.parametrize("prec", [ox.FP64, ox.FP32_IR])
 def test_group_of_several_resident_launches(prec):
     """A group with more workgroups than the chip holds, rows of 9 and 27
@@ -100,7 +123,8 @@ def test_group_of_several_resident_launches(prec):
 
 @pytest.mark.parametrize("n,width", [(1, 1), (300, 3), (5000, 27), (5000, 29), (262144, 3),
                                      (262145, 3)])
-def test_noalloc_rows_and_sizes(n, width):
+@pytest.mark.parametrize("method", [ox.CG, ox.BICGSTAB])
+def test_noalloc_rows_and_sizes(n, width, method):
     """Caller-held CRS rows of up to 27 entries run resident, longer ones and
     larger systems do not; twice in a row from the same start, the same bits,
     and the residual they report."""
@@ -117,7 +141,8 @@ def test_noalloc_rows_and_sizes(n, width):
     xs = []
     for _ in range(2):
         x = DevArray(np.zeros(n))
-        info, _ = ox.solve_crs_noalloc(n, *(d.ptr for d in dev), x.ptr, tol=1e-12, max_iter=500)
+        info, _ = ox.solve_crs_noalloc(n, *(d.ptr for d in dev), x.ptr, tol=1e-12, max_iter=500,
+                                       method=method)
         assert info["converged"] == 1
         xs.append(x.get())
     assert np.array_equal(*xs)
