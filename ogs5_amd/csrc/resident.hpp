@@ -52,6 +52,7 @@ constexpr int kStreamVb = 4;
 constexpr int kStreamBlocks = 1024;
 constexpr int kStreamSlots = 9;
 constexpr int kStreamMaxRows = kStreamBlocks * kStreamSlots * kBlock;
+constexpr int kFirstPoll = 12;                // 64-clock units before the first poll
 constexpr unsigned kResPolls = 1u << 21;      // polls of one wait (seconds)
 constexpr long long kCensusTicks = 20000;     // 100 MHz: 200 us
 constexpr int kCensusRing = 64;
@@ -229,6 +230,11 @@ struct ResExchange {
         }
         meanwhile();
         if (wave < 4) {
+            // the others' sums arrive no sooner: polls before then only slow
+            // the stores they wait for (200 x 200 quads FP64 4.40 -> 4.08 ms;
+            // a pause twice as long, pauses between polls, or several polls
+            // under way at once are slower again)
+            __builtin_amdgcn_s_sleep(kFirstPoll);
             unsigned long long got[NV];
 #pragma unroll
             for (int k = 0; k < NV; k++) got[k] = 0;
