@@ -348,9 +348,55 @@ __device__ __forceinline__ T at_byte(const OGSX_GL T* base, unsigned off)
     return *(const OGSX_GL T*)((const OGSX_GL char*)base + off);
 }
 
+// Row `row` of the FP64 matrix times the FP64 vector that the workgroups have
+// published in x, as k_ir_residual sums it (the symmetric diagonal copy in CRS
+// order, or the CRS row).
+__device__ __forceinline__ double row_times_published(const SysDev& S, int row,
+                                                      const OGSX_GL double* x)
+{
+#pragma clang fp contract(off)
+    double s = 0.0;
+    if (gl(S.prm)->dia) {
+        const OGSX_GL double* dv = gl(S.m64.dia_val);
+        const OGSX_GL int* off = gl(S.m64.dia_off);
+        const int K = S.m64.dia_k, n = S.n;
+#pragma unroll 4
+        for (int k = K - 1; k >= 0; k--) {
+            const int lo = max(row - off[k], 0);
+            const double a = dv[(int64_t)(k + 1) * n + lo], xl = agent_load(x + lo);
+            const double prod = (row >= off[k] ? a : 0.0) * xl;
+            s = s + prod;
+        }
+        const double prod = dv[row] * agent_load(x + row);
+        s = s + prod;
+#pragma unroll 4
+        for (int k = 0; k < K; k++) {
+            const double a = dv[(int64_t)(k + 1) * n + row];
+            const double prod = a * agent_load(x + min(row + off[k], n - 1));
+            s = s + prod;
+        }
+    } else {
+        const OGSX_GL int* cols = gl(S.m64.col);
+        const OGSX_GL double* A = gl(S.A);
+        const int k1 = gl(S.m64.ptr)[row + 1];
+#pragma unroll 4
+        for (int k = gl(S.m64.ptr)[row]; k < k1; k++) {
+            const double prod = A[k] * agent_load(x + cols[k]);
+            s = s + prod;
+        }
+    }
+    return s;
+}
+
 // A batch of Jacobi-CG iterations (k_cg_spmv, k_cg_update, k_cg_direction)
 // of the members of `g`, one row per thread.  What bounds it: the two
 // exchanges, 1.4-2 us each, and one gather of z.
+//
+// FP32 (inside FP64 refinement with reliable updates): a recurrence that stops
+// for an update or at its target goes through the refinement step right here
+// (k_ir_fold, k_ir_residual, k_ir_decide, k_ir_prepare, k_cg_rescan,
+// k_cg_resume, in their arithmetic) and runs on; only a finished solve or the
+// batch's end leaves the launch.
 template <typename T, int NE, bool PAIR, int VB>
 __global__ __launch_bounds__(kBlock * VB) void k_cg_resident(Grp g, ResLaunch L)
 {
@@ -367,7 +413,11 @@ __global__ __launch_bounds__(kBlock * VB) void k_cg_resident(Grp g, ResLaunch L)
     const int G = S.G, n = S.n, tid = threadIdx.x;
     const int it0 = st->iter, max_iter = st->max_iter;
     const double bnorm = st->bnorm;
-    const double tol = gl(S.prm)->tol, upd_thresh = gl(S.prm)->upd_thresh;
+    double tol = gl(S.prm)->tol, upd_thresh = gl(S.prm)->upd_thresh;
+    constexpr bool IR = sizeof(T) == 4;
+    const bool reliable = IR && gl(S.prm)->ir_reliable;
+    int updates = 0, status = -1;
+    double ir_error = 0.0, maxr = 0.0;
     double rr = st->rr;
     ResExchange<VB> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, G / VB,
                        sw, sm, &ok};
@@ -404,7 +454,8 @@ __global__ __launch_bounds__(kBlock * VB) void k_cg_resident(Grp g, ResLaunch L)
         const T alpha = (T)alpha_d;
         x = x + alpha * p;
         r = r - alpha * s;
-        const T zi = r / d;
+        T zi = r / d;
+        bool limit = true;  // (k_cg_direction tests the limit, k_cg_resume does not)
         if (have) agent_store(z + row, zi);
         double two[2] = {have ? (double)r * (double)r : 0.0, have ? (double)zi * (double)r : 0.0};
         double res[2];
@@ -415,7 +466,45 @@ __global__ __launch_bounds__(kBlock * VB) void k_cg_resident(Grp g, ResLaunch L)
         it++;
         if (error < tol || rnorm < upd_thresh) {
             done = error < tol ? 1 : 5;
-            break;
+            if constexpr (!IR) break;
+            if (!reliable) break;
+            // x64 += unscale x32; r64 = b - A x64
+            const OGSX_GL KrylovParams* P = gl(S.prm);
+            OGSX_GL double* x64 = wave_uniform(gl(S.v64.x));
+            const double bi = gl(S.v64.b)[row];
+            if (have) agent_store(x64 + row, agent_load(x64 + row) + P->unscale * (double)x);
+            good = ex.barrier([] {});
+            if (!good) break;
+            const double ri = bi - row_times_published(S, row, x64);
+            double norms[1] = {have ? ri * ri : 0.0}, rs[1];
+            good = ex.sum(norms, rs);
+            if (!good) break;
+            // the decision of k_ir_decide, in every workgroup
+            const double rn = sqrt(rs[0]);
+            updates++;
+            ir_error = rn / gl(S.irs)->bnorm;
+            if (ir_error < P->ir_tol) {
+                status = 1;
+                break;
+            }
+            if (it >= P->ir_max_iter) {
+                status = 0;
+                break;
+            }
+            maxr = rn * P->scale;
+            upd_thresh = P->ir_delta * maxr;
+            tol = P->ir_tol * gl(S.irs)->bnorm * P->scale * (rn / rn);
+            // the recurrence resumes from the true residual
+            done = 0;
+            r = (T)(ri * P->scale);
+            x = 0;
+            zi = r / d;
+            if (have) agent_store(z + row, zi);
+            two[0] = have ? (double)r * (double)r : 0.0;
+            two[1] = have ? (double)zi * (double)r : 0.0;
+            good = ex.sum(two, res);
+            if (!good) break;
+            limit = false;
         }
         const T beta = (T)(res[1] / rr_old);
 #pragma unroll
@@ -434,7 +523,7 @@ __global__ __launch_bounds__(kBlock * VB) void k_cg_resident(Grp g, ResLaunch L)
         }
         p = zi + beta * p;
         rr = res[1];
-        if (it >= max_iter) {
+        if (limit && it >= max_iter) {
             done = 2;
             break;
         }
@@ -453,6 +542,19 @@ __global__ __launch_bounds__(kBlock * VB) void k_cg_resident(Grp g, ResLaunch L)
         st->done = done;
         st->resident = good ? 0 : 2;
         S.rs->phase = ex.set;
+        if (IR && updates > 0) {
+            OGSX_GL IRState* R = gl(S.irs);
+            R->error = ir_error;
+            R->total = it;
+            R->updates = R->updates + updates;
+            R->status = status;
+            R->action = status < 0 ? 2 : 0;
+            if (status < 0) {  // (a finished solve's last decision leaves these)
+                R->maxr = maxr;
+                gl(S.prm)->upd_thresh = upd_thresh;
+                gl(S.prm)->tol = tol;
+            }
+        }
     }
 }
 

@@ -39,7 +39,7 @@ def _scenario(kind, shape, seed=3, permute=False):
 def _solve(sc, system, separate, **kw):
     system[1].profile(separate)
     r = W.run_gpu(sc, system=system, **kw)
-    return r["x"], r["info"][0]
+    return r["x"], r["info"][-1]
 
 
 def _same(a, b):
@@ -80,6 +80,25 @@ def test_cg_rows_read_from_crs(kind, shape, prec):
         system = W.make_system(sc, prec)
         _same(_solve(sc, system, False, dirichlet=bc), _solve(sc, system, True, dirichlet=bc))
         system[1].close()
+
+
+@pytest.mark.parametrize("permute", [False, True])
+@pytest.mark.parametrize("kind,shape", [("line", (300,)), ("quad", (61, 50)), ("quad", (300, 240)),
+                                        ("tet", (9, 8, 10)), ("hex", (14, 11, 13))])
+def test_refinement_steps_in_the_launch(kind, shape, permute):
+    """FP32-IR solves to the tolerance (several reliable updates, taken inside
+    the launch) and to a limit between two of them; FP64 rows from the diagonal
+    copy and from CRS; a second solve on the same system."""
+    sc = _scenario(kind, shape, permute=permute)
+    sc.steps = sc.steps * 2
+    system = W.make_system(sc, ox.FP32_IR)
+    for max_iter in (5000, 37):
+        sc.max_iter = max_iter
+        got = _solve(sc, system, False)
+        _same(got, _solve(sc, system, True))
+        assert got[1]["converged"] == (max_iter == 5000)
+        assert max_iter != 5000 or got[1]["outer"] >= 2  # updates, the last one final
+    system[1].close()
 
 
 # sizes as above; the largest resident system of 256-thread workgroups
