@@ -93,6 +93,7 @@ __device__ __forceinline__ double lanes_down(double v)
 // the serial path of every dot product.
 __device__ __forceinline__ double wave_sum(double v)
 {
+#pragma clang fp contract(off)  // v may be a product: rounded before it is added
     v += lanes_down<32>(v);
     v += lanes_down<16>(v);
     v += lanes_down<8>(v);

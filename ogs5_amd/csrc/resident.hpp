@@ -726,6 +726,341 @@ __global__ __launch_bounds__(kBlock * VB) void k_bi_resident(Grp g, ResLaunch L)
     }
 }
 
+// ---- Systems of one workgroup -------------------------------------------------
+// The smallest systems (FP64, up to 2048 rows) fit one workgroup of W waves:
+// wave i takes the 64-row slices i, i + W, ..., up to ROWS of them, with their
+// matrix entries in registers and every vector in LDS.  Nothing is exchanged
+// through memory; a dot product costs one workgroup barrier (0.1 us instead of
+// 1.4-2).  Instruction issue bounds these kernels, so the waves are few and the
+// rows per thread several.  Chunks of these sizes have one row per thread, so a
+// slice's sum is one wave's sum of store_partials, and the sums below add up in
+// its order.
+constexpr int kOneMaxSlices = 32;
+
+struct OneSums {
+    double (*ws)[kSlotVals][kOneMaxSlices];  // [2]: slice sums, by turns
+    int turn, G, ns;
+
+    template <int W, int NV, int ROWS>
+    __device__ __forceinline__ void sum(const double (&v)[ROWS][NV], double (&out)[NV])
+    {
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+        for (int j = 0; j < ROWS; j++)
+#pragma unroll
+            for (int k = 0; k < NV; k++) {
+                const double s = wave_sum(v[j][k]);
+                if (lane == 0) ws[turn][k][wave + W * j] = s;
+            }
+        __syncthreads();
+        // chunk `lane`: its slices' sums, then the sum over the chunks
+        const int sb = lane < G ? ns * lane / G : 0, se = lane < G ? ns * (lane + 1) / G : 0;
+#pragma unroll
+        for (int k = 0; k < NV; k++) {
+            double c[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) c[i] = ws[turn][k][min(sb + i, kOneMaxSlices - 1)];
+            double s = sb < se ? c[0] : 0.0;
+#pragma unroll
+            for (int i = 1; i < 4; i++) s += sb + i < se ? c[i] : 0.0;
+            const double t = wave_sum(s);
+            const long long b = __double_as_longlong(t);
+            const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)b);
+            const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(b >> 32));
+            out[k] = __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+        }
+        turn ^= 1;  // (a wave is at most one sum ahead of another)
+    }
+};
+
+// A thread's rows: entries, and their columns' byte offsets into an LDS vector
+// two to a register (up to 16 KB a vector).
+template <int NE, int ROWS, int W>
+struct OneRows {
+    double a[ROWS][NE];
+    unsigned col[ROWS][(NE + 1) / 2];
+
+    __device__ __forceinline__ void load(const SysDev& S)
+    {
+#pragma unroll
+        for (int j = 0; j < ROWS; j++) {
+            const int row = (int)threadIdx.x + 64 * W * j;
+            unsigned c[NE];
+            load_row<double, NE, false>(S, gl(S.prm)->dia, min(row, S.n - 1), a[j], c);
+#pragma unroll
+            for (int e = 0; e < (NE + 1) / 2; e++)
+                col[j][e] = c[2 * e] | (2 * e + 1 < NE ? c[2 * e + 1] << 16 : 0u);
+        }
+    }
+    __device__ __forceinline__ double sum(int j, const double* x) const
+    {
+        double v[NE];
+#pragma unroll
+        for (int e = 0; e < NE; e++) {
+            const unsigned off = e & 1 ? col[j][e / 2] >> 16 : col[j][e / 2] & 0xffffu;
+            v[e] = *(const double*)((const char*)x + off);
+        }
+        return row_sum<double, NE, false>(a[j], v);
+    }
+};
+
+// Jacobi-CG of one-workgroup members (the recurrence of k_cg_resident).
+template <int NE, int ROWS, int W>
+__global__ __launch_bounds__(64 * W) void k_cg_one(Grp g, ResLaunch L)
+{
+    extern __shared__ __align__(16) char stream_lds[];
+    __shared__ double ws[2][kSlotVals][kOneMaxSlices];
+    const SysDev& S = g.sys[g.blk2sys ? g.blk2sys[blockIdx.x] : 0];
+    OGSX_GL KrylovState* st = gl(S.st);
+    if (st->done) return;
+    const int n = S.n, tid = threadIdx.x;
+    const int it0 = st->iter, max_iter = st->max_iter;
+    const double bnorm = st->bnorm;
+    const double tol = gl(S.prm)->tol, upd_thresh = gl(S.prm)->upd_thresh;
+    double rr = st->rr, error = st->error, alpha = st->alpha, rr_old = st->rr_old;
+    OneSums sums{ws, 0, S.G, (n + 63) / 64};
+    const GVec<double> v = gvec(S.v64);
+    constexpr int N = 64 * W * ROWS;
+    double* const pl = (double*)stream_lds;  // by row; the others by thread
+    double* const xl = pl + N;
+    double* const rl = xl + N;
+    double* const dl = rl + N;
+    OneRows<NE, ROWS, W> rows;
+    rows.load(S);
+#pragma unroll
+    for (int j = 0; j < ROWS; j++) {
+        const int row = tid + 64 * W * j;
+        const bool have = row < n;
+        pl[row] = have ? v.p[row] : 0.0;
+        xl[row] = have ? v.x[row] : 0.0;
+        rl[row] = have ? v.r[row] : 0.0;
+        dl[row] = have ? v.d[row] : 1.0;
+    }
+    int it = it0, done = 0;
+    for (int k = 0; k < L.iters; k++) {
+        __syncthreads();  // p is written
+        double s[ROWS], dot[ROWS][1], ps[1];
+#pragma unroll
+        for (int j = 0; j < ROWS; j++) {
+            const int row = tid + 64 * W * j;
+            s[j] = rows.sum(j, pl);
+            dot[j][0] = row < n ? pl[row] * s[j] : 0.0;
+        }
+        sums.sum<W, 1, ROWS>(dot, ps);
+        alpha = rr / ps[0];
+        rr_old = rr;
+        double z[ROWS], two[ROWS][2], res[2];
+#pragma unroll
+        for (int j = 0; j < ROWS; j++) {
+            const int row = tid + 64 * W * j;
+            xl[row] = xl[row] + alpha * pl[row];
+            const double r = rl[row] - alpha * s[j];
+            rl[row] = r;
+            z[j] = r / dl[row];
+            two[j][0] = row < n ? r * r : 0.0;
+            two[j][1] = row < n ? z[j] * r : 0.0;
+        }
+        sums.sum<W, 2, ROWS>(two, res);
+        const double rnorm = sqrt(res[0]);
+        error = rnorm / bnorm;
+        it++;
+        if (error < tol || rnorm < upd_thresh) {
+            done = error < tol ? 1 : 5;
+            break;
+        }
+        const double beta = res[1] / rr_old;
+#pragma unroll
+        for (int j = 0; j < ROWS; j++) {
+            const int row = tid + 64 * W * j;
+            pl[row] = z[j] + beta * pl[row];
+        }
+        rr = res[1];
+        if (it >= max_iter) {
+            done = 2;
+            break;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < ROWS; j++) {
+        const int row = tid + 64 * W * j;
+        if (row < n) {
+            v.x[row] = xl[row];
+            v.r[row] = rl[row];
+            v.p[row] = pl[row];
+        }
+    }
+    if (tid == 0) {
+        st->error = error;
+        st->rr = rr;
+        st->rr_old = rr_old;
+        st->alpha = alpha;
+        st->iter = it;
+        st->done = done;
+        st->resident = 0;
+    }
+}
+
+// BiCGStab of one-workgroup members (the recurrence of k_bi_resident).
+template <int NE, int ROWS, int W>
+__global__ __launch_bounds__(64 * W) void k_bi_one(Grp g, ResLaunch L)
+{
+    extern __shared__ __align__(16) char stream_lds[];
+    __shared__ double ws[2][kSlotVals][kOneMaxSlices];
+    const SysDev& S = g.sys[g.blk2sys ? g.blk2sys[blockIdx.x] : 0];
+    OGSX_GL KrylovState* st = gl(S.st);
+    if (st->done != 0 || st->pend != 0) return;
+    const int n = S.n, tid = threadIdx.x, G = S.G, ns = (n + 63) / 64;
+    const int it0 = st->iter, max_iter = st->max_iter;
+    const double bnorm = st->bnorm;
+    const double tol = gl(S.prm)->tol;
+    double rho0 = st->rho0, rho1 = st->rho1, alpha = st->alpha, omega = st->omega;
+    double error = st->error;
+    OneSums sums{ws, 0, G, ns};
+    const GVec<double> v = gvec(S.v64);
+    constexpr int N = 64 * W * ROWS;
+    double* const hl = (double*)stream_lds;  // preconditioned p, by row
+    double* const tl = hl + N;               // preconditioned s, by row
+    double* const xl = tl + N;               // the others by thread
+    double* const rl = xl + N;
+    double* const pl = rl + N;
+    double* const vl = pl + N;
+    double* const ol = vl + N;
+    double* const dl = ol + N;
+    OneRows<NE, ROWS, W> rows;
+    rows.load(S);
+    double rr[ROWS][2], res[2];
+#pragma unroll
+    for (int j = 0; j < ROWS; j++) {
+        const int row = tid + 64 * W * j;
+        const bool have = row < n;
+        xl[row] = have ? v.x[row] : 0.0;
+        rl[row] = have ? v.r[row] : 0.0;
+        pl[row] = have ? v.p[row] : 0.0;
+        vl[row] = have ? v.v[row] : 0.0;
+        ol[row] = have ? v.r0[row] : 0.0;
+        dl[row] = have ? v.d[row] : 1.0;
+        rr[j][0] = rl[row] * rl[row];
+        rr[j][1] = ol[row] * rl[row];
+    }
+    int it = it0, done = 0, pend = 0;
+    sums.sum<W, 2, ROWS>(rr, res);
+    for (int k = 0; k < L.iters; k++) {
+        if (it > 0) {
+            const double err = sqrt(res[0]) / bnorm;
+            if (err < tol || fabs(omega) < DBL_MIN || it >= max_iter) {
+                error = err;
+                done = err < tol ? 1 : fabs(omega) < DBL_MIN ? 3 : 2;
+                break;
+            }
+        }
+        if (fabs(res[1]) < DBL_MIN) {
+            done = 6;
+            break;
+        }
+        rho1 = res[1];
+        const double beta = it > 0 ? (rho1 / rho0) * (alpha / omega) : 0.0;
+#pragma unroll
+        for (int j = 0; j < ROWS; j++) {
+            const int row = tid + 64 * W * j;
+            const double p = it == 0 ? rl[row] : bi_p(rl[row], beta, pl[row], omega, vl[row]);
+            pl[row] = p;
+            hl[row] = p / dl[row];
+        }
+        it++;
+        __syncthreads();
+        double one[ROWS][1], rv[1];
+#pragma unroll
+        for (int j = 0; j < ROWS; j++) {
+            const int row = tid + 64 * W * j;
+            const double vi = row < n ? rows.sum(j, hl) : 0.0;
+            vl[row] = vi;
+            one[j][0] = ol[row] * vi;
+        }
+        sums.sum<W, 1, ROWS>(one, rv);
+        alpha = rho1 / rv[0];
+        rho0 = rho1;
+        double s[ROWS], t[ROWS], three[ROWS][3], out[3];
+#pragma unroll
+        for (int j = 0; j < ROWS; j++) {
+            const int row = tid + 64 * W * j;
+            s[j] = rl[row] - alpha * vl[row];
+            tl[row] = s[j] / dl[row];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < ROWS; j++) {
+            const int row = tid + 64 * W * j;
+            t[j] = row < n ? rows.sum(j, tl) : 0.0;
+            three[j][0] = s[j] * s[j];
+            three[j][1] = t[j] * t[j];
+            three[j][2] = t[j] * s[j];
+        }
+        sums.sum<W, 3, ROWS>(three, out);
+        const double err = sqrt(out[0]) / bnorm;
+        if (err < tol) {
+#pragma unroll
+            for (int j = 0; j < ROWS; j++) {
+                const int row = tid + 64 * W * j;
+                xl[row] = xl[row] + alpha * hl[row];
+            }
+            error = err;
+            pend = 1;
+            break;
+        }
+        omega = (out[1] > DBL_MIN) ? out[2] / out[1] : 1.0;
+#pragma unroll
+        for (int j = 0; j < ROWS; j++) {
+            const int row = tid + 64 * W * j;
+            xl[row] = bi_x(xl[row], alpha, hl[row], omega, tl[row]);
+            const double r = s[j] - omega * t[j];
+            rl[row] = r;
+            rr[j][0] = row < n ? r * r : 0.0;
+            rr[j][1] = row < n ? ol[row] * r : 0.0;
+        }
+        sums.sum<W, 2, ROWS>(rr, res);
+    }
+#pragma unroll
+    for (int j = 0; j < ROWS; j++) {
+        const int row = tid + 64 * W * j;
+        if (row < n) {
+            v.x[row] = xl[row];
+            v.r[row] = rl[row];
+            v.p[row] = pl[row];
+            v.v[row] = vl[row];
+        }
+    }
+    // (r, r) and (r0, r) of the last update, for a direction launched separately
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < ROWS; j++)
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const double w = wave_sum(rr[j][k]);
+            if ((tid & 63) == 0) ws[0][k][(tid >> 6) + W * j] = w;
+        }
+    __syncthreads();
+    if (tid < G) {
+        const int sb = ns * tid / G, se = ns * (tid + 1) / G;
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            double s = 0.0;
+            for (int i = sb; i < se; i++) s = i == sb ? ws[0][k][i] : s + ws[0][k][i];
+            gl(S.part)[k * part_stride(G) + tid] = s;  // (G is 8: q = 1)
+        }
+    }
+    if (tid == 0) {
+        st->error = error;
+        st->rho0 = rho0;
+        st->rho1 = rho1;
+        st->alpha = alpha;
+        st->omega = omega;
+        st->iter = it;
+        st->pend = pend;
+        st->done = done;
+        st->resident = 0;
+    }
+}
+
 // The symmetric diagonal copy as k_cg_stream reads it: KC offsets and every
 // array's base in scalar registers.
 template <int KC, typename T>
@@ -1055,6 +1390,7 @@ constexpr size_t stream_vec_bytes(int n, int G, size_t size)
     const int ns = (n + 63) / 64;
     return (size_t)(((ns + G - 1) / G * 64 + kBlock - 1) / kBlock) * kBlock * kStreamVb * size;
 }
-constexpr size_t kStreamLds = 160 * 1024 - 1024;  // a compute unit's, less the exchange's
+constexpr int kCuLds = 160 * 1024;             // LDS of a compute unit
+constexpr size_t kStreamLds = kCuLds - 1024;  // ... less the exchange's
 
 }  // namespace ogsx

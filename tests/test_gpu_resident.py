@@ -51,8 +51,12 @@ def _same(a, b):
 # sizes: one row; a chunk and one row more; the partial sums' q = 1, 2 and 4
 # neighbours per thread; the largest resident system of each row length and
 # the next one up
-CG = [("line", (1,)), ("line", (255,)), ("line", (256,)), ("line", (2047,)), ("line", (2048,)),
-      ("quad", (1, 1)), ("quad", (33, 21)), ("quad", (255, 255)), ("quad", (256, 255)),
+# (FP64 also: one workgroup, of 256, 1024 and 2048 rows, and one row more)
+CG = [("line", (1,)), ("line", (255,)), ("line", (256,)), ("line", (1023,)), ("line", (1024,)),
+      ("line", (2047,)), ("line", (2048,)), ("line", (4096,)),
+      ("quad", (1, 1)), ("quad", (33, 21)), ("quad", (63, 31)), ("quad", (64, 63)),
+      ("tet", (3, 7, 7)), ("hex", (3, 7, 7)),
+      ("tet", (11, 12, 11)), ("tet", (12, 12, 12)), ("hex", (9, 9, 9)), ("hex", (10, 9, 9)), ("quad", (255, 255)), ("quad", (256, 255)),
       ("quad", (361, 362)), ("quad", (511, 511)), ("quad", (512, 511)),
       ("tet", (1, 1, 1)), ("tet", (9, 7, 5)), ("tet", (50, 50, 49)), ("tet", (50, 50, 50)),
       ("hex", (1, 1, 1)), ("hex", (9, 7, 5)), ("hex", (50, 50, 49)), ("hex", (50, 50, 50))]
@@ -103,7 +107,9 @@ def test_refinement_steps_in_the_launch(kind, shape, permute):
 
 # sizes as above; the largest resident system of 256-thread workgroups
 # (65,536 rows) and of 512-thread ones (131,072) and the next one up
-BI = [("line", (1,)), ("line", (255,)), ("line", (2048,)), ("quad", (1, 1)), ("quad", (33, 21)),
+BI = [("line", (1,)), ("line", (255,)), ("line", (1023,)), ("line", (1024,)), ("line", (2047,)),
+      ("line", (2048,)), ("quad", (1, 1)), ("quad", (33, 21)), ("tet", (9, 9, 9)),
+      ("tet", (10, 9, 9)), ("hex", (9, 9, 9)), ("hex", (10, 9, 9)),
       ("quad", (361, 361)), ("quad", (361, 362)), ("tet", (1, 1, 1)), ("tet", (9, 7, 5)),
       ("tet", (39, 39, 39)), ("tet", (40, 40, 40)), ("tet", (50, 50, 50)),
       ("hex", (1, 1, 1)), ("hex", (9, 7, 5)), ("hex", (39, 39, 39)), ("hex", (40, 40, 40))]
@@ -140,7 +146,7 @@ def test_group_of_several_resident_launches(prec):
         system[1].close()
 
 
-@pytest.mark.parametrize("n,width", [(1, 1), (300, 3), (5000, 27), (5000, 29), (262144, 3),
+@pytest.mark.parametrize("n,width", [(1, 1), (300, 3), (2048, 9), (2049, 9), (5000, 27), (5000, 29), (262144, 3),
                                      (262145, 3)])
 @pytest.mark.parametrize("method", [ox.CG, ox.BICGSTAB])
 def test_noalloc_rows_and_sizes(n, width, method):
