@@ -1384,6 +1384,283 @@ __global__ __launch_bounds__(kBlock * kStreamVb) void k_cg_stream(Grp g, ResLaun
     }
 }
 
+// A SELL-64 matrix with a stencil dictionary as k_bi_stream reads it: the
+// dictionary in LDS, a row's pattern kept by its thread.
+template <typename T>
+struct DictRows {
+    const OGSX_GL T* val;
+    const OGSX_GL int* ptr;
+    const OGSX_GL int* width;
+    const int* delta;
+
+    // Row sum of the thread's row in slice `slice`, in CRS order, U entries at
+    // a time: their loads are issued together, those past the row's width read
+    // its last entry again and are not added (the width is the wave's).
+    __device__ __forceinline__ T sum(const OGSX_GL T* x, int slice, int row, int pat, int n) const
+    {
+#pragma clang fp contract(off)
+        constexpr int U = sizeof(T) == 4 ? 16 : 8;
+        const int w = __builtin_amdgcn_readfirstlane(width[slice]);
+        const int base = __builtin_amdgcn_readfirstlane(ptr[slice]);
+        const int lane = (int)threadIdx.x & 63;
+        T s = 0;
+        for (int e0 = 0; e0 < w; e0 += U) {
+            T a[U], xv[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int e = min(e0 + u, w - 1);
+                a[u] = at_byte(val, (unsigned)(base + e * 64 + lane) * sizeof(T));
+                xv[u] = at_byte(x, (unsigned)(min(row, n - 1) + delta[pat + e]) * sizeof(T));
+            }
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (e0 + u < w) {
+                    const T prod = a[u] * xv[u];
+                    s = s + prod;
+                }
+        }
+        return s;
+    }
+};
+
+// BiCGStab of one system too large for a thread per row (the recurrence of
+// k_bi_resident, the layout of k_cg_stream: vectors in LDS, up to ROWS rows per
+// thread, the matrix streamed).  The preconditioned p and s are published into
+// four vectors in turn and gathered through the caches, which are invalidated
+// once in two iterations.  Five exchanges per iteration: the new p (a barrier),
+// (r0, v), (s, s) with the new s, (t, t) and (t, s), (r, r) and (r0, r).
+// The matrix read twice per iteration and the five exchanges bound it: the
+// FP32 steps of 80x72x64 hexes cut into tets (385,000 rows, 15 entries) take
+// 25 us per iteration, 37 us with a launch per phase; a time step of it 4.31 ->
+// 2.56 ms.
+template <typename T, int ROWS>
+__global__ __launch_bounds__(kBlock * kStreamVb) void k_bi_stream(Grp g, ResLaunch L)
+{
+    constexpr int VB = kStreamVb, NT = kBlock * VB;
+    extern __shared__ __align__(16) char stream_lds[];
+    __shared__ double sw[kSlotVals][4 * VB];
+    __shared__ double sm[kSlotVals][4];
+    __shared__ int flag, ok;
+    const int si = g.blk2sys ? g.blk2sys[blockIdx.x] : 0;
+    const int launched = (int)blockIdx.x - (g.blk2sys ? g.blk0[si] : 0);
+    const SysDev& S = g.sys[si];
+    OGSX_GL KrylovState* st = gl(S.st);
+    const bool idle = st->done != 0 || st->pend != 0;
+    const int G = S.G, n = S.n, tid = threadIdx.x, nwg = G / VB;
+    const int w = nwg % kNumXcd ? launched
+                                : (launched % kNumXcd) * (nwg / kNumXcd) + launched / kNumXcd;
+    const int it0 = st->iter, max_iter = st->max_iter;
+    const double bnorm = st->bnorm;
+    const double tol = gl(S.prm)->tol;
+    double rho0 = st->rho0, rho1 = st->rho1, alpha_d = st->alpha, omega_d = st->omega;
+    double error = st->error;
+    ResExchange<VB> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, nwg, sw, sm, &ok};
+    if (tid == 0) ok = 1;
+    if (!res_census(L, idle, &flag)) {
+        if (!idle && w == 0 && tid == 0) st->resident = 1;
+        return;
+    }
+    const MatView<T>& M = mv_of<T>(S);
+    const GVec<T> v = gvec(kv_of<T>(S));
+    OGSX_GL T* const vd = wave_uniform(v.d);
+    const int c = w * VB + tid / kBlock, ns = (n + 63) / 64;
+    const int beg = (int)((int64_t)ns * c / G) * 64;
+    const int end = min((int)((int64_t)ns * (c + 1) / G) * 64, n);
+    const int first = beg + chunk_thread();
+    // vector q of row first + 256 j at [(q ROWS + j) 1024 + tid]; then the
+    // dictionary
+    T* const rl = (T*)stream_lds + tid;  // r, and s
+    T* const pl = rl + ROWS * NT;
+    T* const vl = pl + ROWS * NT;
+    T* const xl = vl + ROWS * NT;
+    T* const ol = xl + ROWS * NT;        // r0
+    T* const hl = ol + ROWS * NT;        // preconditioned p
+    T* const kl = hl + ROWS * NT;        // preconditioned s
+    T* const tl = kl + ROWS * NT;        // t
+    int* const delta = (int*)((T*)stream_lds + 8 * ROWS * NT);
+    for (int i = tid; i < M.pat_cnt * M.pat_w; i += NT) delta[i] = gl(M.pat_delta)[i];
+    const DictRows<T> m{wave_uniform(gl(const_cast<T*>(M.sval))),
+                        wave_uniform(gl(const_cast<int*>(M.sell_ptr))),
+                        wave_uniform(gl(const_cast<int*>(M.sell_w))), delta};
+    int pat[ROWS];
+    T dj[ROWS];
+#pragma unroll
+    for (int j = 0; j < ROWS; j++) {
+        const int i = first + j * kBlock;
+        pat[j] = 0;
+        dj[j] = 1;
+        if (i < end) {
+            pat[j] = (int)gl(M.sell_pid)[i] * M.pat_w;
+            dj[j] = vd[i];
+            rl[j * NT] = v.r[i];
+            pl[j * NT] = v.p[i];
+            vl[j * NT] = v.v[i];
+            xl[j * NT] = v.x[i];
+            ol[j * NT] = v.r0[i];
+        }
+    }
+    OGSX_GL T* const ring[4] = {wave_uniform(v.ph), wave_uniform(v.sh), wave_uniform(v.s),
+                                wave_uniform(v.t)};
+    auto row_sums = [&](const OGSX_GL T* x, T* to) {
+#pragma unroll
+        for (int j = 0; j < ROWS; j++) {
+            int i = first + j * kBlock;
+            asm("" : "+v"(i));
+            if (i < end) to[j * NT] = m.sum(x, __builtin_amdgcn_readfirstlane(i >> 6), i, pat[j], n);
+        }
+    };
+    int it = it0, done = 0, pend = 0;
+    double rr[2] = {0.0, 0.0}, res[2];
+#pragma unroll
+    for (int j = 0; j < ROWS; j++)
+        if (first + j * kBlock < end) {
+            const double r = (double)rl[j * NT];
+            rr[0] = fma(r, r, rr[0]);
+            rr[1] = fma((double)ol[j * NT], r, rr[1]);
+        }
+    bool good = ex.sum(rr, res);
+    for (int k = 0; good && k < L.iters; k++) {
+        if (it > 0) {
+            const double err = sqrt(res[0]) / bnorm;
+            if (err < tol || fabs(omega_d) < DBL_MIN || it >= max_iter) {
+                error = err;
+                done = err < tol ? 1 : fabs(omega_d) < DBL_MIN ? 3 : 2;
+                break;
+            }
+        }
+        if (fabs(res[1]) < DBL_MIN) {
+            done = 6;
+            break;
+        }
+        rho1 = res[1];
+        T beta = 0, omega = 0;
+        if (it > 0) {
+            beta = (T)((rho1 / rho0) * (alpha_d / omega_d));
+            omega = (T)omega_d;
+        }
+        OGSX_GL T* const hp = k & 1 ? ring[2] : ring[0];
+        OGSX_GL T* const hs = k & 1 ? ring[3] : ring[1];
+#pragma unroll
+        for (int j = 0; j < ROWS; j++) {
+            const int i = first + j * kBlock;
+            if (i < end) {
+                const T p = it == 0 ? rl[j * NT]
+                                    : bi_p(rl[j * NT], beta, pl[j * NT], omega, vl[j * NT]);
+                pl[j * NT] = p;
+                const T h = p / dj[j];
+                hl[j * NT] = h;
+                agent_store(hp + i, h);
+            }
+        }
+        it++;
+        good = ex.barrier([] {});
+        if (!good) break;
+        if ((k & 1) == 0) {
+            if (tid < 64) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            __syncthreads();
+        }
+        row_sums(hp, vl);
+        double one[1] = {0.0}, rv[1];
+#pragma unroll
+        for (int j = 0; j < ROWS; j++)
+            if (first + j * kBlock < end) one[0] = fma((double)ol[j * NT], (double)vl[j * NT], one[0]);
+        good = ex.sum(one, rv);
+        if (!good) break;
+        alpha_d = rho1 / rv[0];
+        rho0 = rho1;
+        const T alpha = (T)alpha_d;
+        double ss[1] = {0.0}, norm[1];
+#pragma unroll
+        for (int j = 0; j < ROWS; j++) {
+            const int i = first + j * kBlock;
+            if (i < end) {
+                const T s = rl[j * NT] - alpha * vl[j * NT];
+                tl[j * NT] = s;  // (t's place until r has been tested and replaced)
+                const T h = s / dj[j];
+                kl[j * NT] = h;
+                agent_store(hs + i, h);
+                ss[0] = fma((double)s, (double)s, ss[0]);
+            }
+        }
+        good = ex.sum(ss, norm);
+        if (!good) break;
+        const double err = sqrt(norm[0]) / bnorm;
+        if (err < tol) {
+#pragma unroll
+            for (int j = 0; j < ROWS; j++)
+                if (first + j * kBlock < end) xl[j * NT] = xl[j * NT] + alpha * hl[j * NT];
+            error = err;
+            pend = 1;
+            break;
+        }
+#pragma unroll
+        for (int j = 0; j < ROWS; j++) rl[j * NT] = tl[j * NT];  // s
+        row_sums(hs, tl);
+        double two[2] = {0.0, 0.0}, sums[2];
+#pragma unroll
+        for (int j = 0; j < ROWS; j++)
+            if (first + j * kBlock < end) {
+                const T t = tl[j * NT];
+                two[0] = fma((double)t, (double)t, two[0]);
+                two[1] = fma((double)t, (double)rl[j * NT], two[1]);
+            }
+        good = ex.sum(two, sums);
+        if (!good) break;
+        omega_d = (sums[0] > DBL_MIN) ? sums[1] / sums[0] : 1.0;
+        omega = (T)omega_d;
+        rr[0] = rr[1] = 0.0;
+#pragma unroll
+        for (int j = 0; j < ROWS; j++)
+            if (first + j * kBlock < end) {
+                xl[j * NT] = bi_x(xl[j * NT], alpha, hl[j * NT], omega, kl[j * NT]);
+                const T r = rl[j * NT] - omega * tl[j * NT];
+                rl[j * NT] = r;
+                rr[0] = fma((double)r, (double)r, rr[0]);
+                rr[1] = fma((double)ol[j * NT], (double)r, rr[1]);
+            }
+        good = ex.sum(rr, res);
+    }
+    const GVec<T> out = gvec(kv_of<T>(S));
+#pragma unroll
+    for (int j = 0; j < ROWS; j++) {
+        const int i = first + j * kBlock;
+        if (i < end) {
+            out.x[i] = xl[j * NT];
+            out.r[i] = rl[j * NT];
+            out.p[i] = pl[j * NT];
+            out.v[i] = vl[j * NT];
+        }
+    }
+    // (r, r) and (r0, r) of the last update, for a direction launched separately
+    OGSX_GL double* part = gl(S.part);
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const double s = wave_sum(rr[k]);
+        if ((tid & 63) == 0) sw[k][tid >> 6] = s;
+    }
+    __syncthreads();
+    if (tid % kBlock == 0) {
+        const int q = part_q(G), vb = tid / kBlock;
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+            part[k * part_stride(G) + kBlock * (c % q) + c / q] =
+                ((sw[k][4 * vb] + sw[k][4 * vb + 1]) + sw[k][4 * vb + 2]) + sw[k][4 * vb + 3];
+    }
+    if (w == 0 && tid == 0) {
+        st->error = error;
+        st->rho0 = rho0;
+        st->rho1 = rho1;
+        st->alpha = alpha_d;
+        st->omega = omega_d;
+        st->iter = it;
+        st->pend = pend;
+        st->done = done;
+        st->resident = good ? 0 : 2;
+        S.rs->phase = ex.set;
+    }
+}
+
 // Bytes of LDS that one vector of k_cg_stream takes.
 constexpr size_t stream_vec_bytes(int n, int G, size_t size)
 {

@@ -112,7 +112,9 @@ BI = [("line", (1,)), ("line", (255,)), ("line", (1023,)), ("line", (1024,)), ("
       ("tet", (10, 9, 9)), ("hex", (9, 9, 9)), ("hex", (10, 9, 9)),
       ("quad", (361, 361)), ("quad", (361, 362)), ("tet", (1, 1, 1)), ("tet", (9, 7, 5)),
       ("tet", (39, 39, 39)), ("tet", (40, 40, 40)), ("tet", (50, 50, 50)),
-      ("hex", (1, 1, 1)), ("hex", (9, 7, 5)), ("hex", (39, 39, 39)), ("hex", (40, 40, 40))]
+      ("hex", (1, 1, 1)), ("hex", (9, 7, 5)), ("hex", (39, 39, 39)), ("hex", (40, 40, 40)),
+      # past a thread per row: 1, 2 and 4 rows per thread
+      ("quad", (600, 440)), ("tet", (64, 64, 64)), ("quad", (1000, 600))]
 
 
 @pytest.mark.parametrize("prec", [ox.FP64, ox.FP32_IR])
