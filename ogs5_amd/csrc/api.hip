@@ -161,6 +161,7 @@ struct ogsx_system {
     const PatternLayout* lay = nullptr;
     std::vector<std::pair<int, double>> tune_log;  // (format, ms) of the last tuning
     size_t tune_n64 = 0;      // leading FP64 entries of tune_log (then FP32)
+    bool fmt_default = false;  // fmt64 / fmt32 hold the format of untimed solves
     bool fmt_forced = false;  // formats set by ogsx_set_spmv_variant
     // SELL-64 copy of the matrix (values refreshed from A when A changed)
     int n_slices = 0;
@@ -872,13 +873,34 @@ int tune_one(ogsx_system* s, int* fmt_out)
 
 int autotune(ogsx_system* s)
 {
-    if (s->fmt64 == 0) {
+    // what the tuner finds goes where the diagonal copy keeps it, if that
+    // stands in for an untimed format
+    int* f64 = s->fmt64 == kFmtSymDia ? &s->fmt64_tuned : &s->fmt64;
+    int* f32 = s->fmt32 == kFmtSymDia ? &s->fmt32_tuned : &s->fmt32;
+    if (s->fmt_default) *f64 = *f32 = 0;
+    s->fmt_default = false;
+    if (*f64 == 0) {
         s->tune_log.clear();
-        OK_TRY((tune_one<double, double>(s, &s->fmt64)));
+        OK_TRY((tune_one<double, double>(s, f64)));
         s->tune_n64 = s->tune_log.size();
     }
-    if (s->precision == OGSX_FP32_IR && s->fmt32 == 0) OK_TRY((tune_one<float, float>(s, &s->fmt32)));
+    if (s->precision == OGSX_FP32_IR && *f32 == 0) OK_TRY((tune_one<float, float>(s, f32)));
     return OGSX_OK;
+}
+
+// A solve that reads none of the tuned formats iteration by iteration (it runs
+// in resident launches, or on the diagonal copy) leaves the tuner's 75 launches
+// out: 0.5 ms of a first solve of 3,900 rows that takes 0.7 ms without them.
+// What it still reads through a format (the FP64 residual of a refinement, the
+// launches after a resident one that found the chip taken) takes this one; it
+// is tuned when a call asks for it.  The choice never changes a result.
+void untimed_format(ogsx_system* s)
+{
+    if (s->fmt64 != 0) return;
+    const int f = s->pat_ok ? kFmtSellPat8C : s->sell16 ? kFmtSell16U8 : kFmtSell32;
+    s->fmt64 = f;
+    s->fmt32 = s->precision == OGSX_FP32_IR ? f : 0;
+    s->fmt_default = true;
 }
 
 double spmv_bytes(const ogsx_system* s, int fmt, int sval, int sx)
@@ -2376,7 +2398,7 @@ int ogsx_set_spmv_variant(ogsx_system* s, int lanes_per_row)
     if (s->sc.active) return fail(OGSX_ESTATE, "system has a solve in progress");
     if (lanes_per_row == 0) {
         s->fmt64 = s->fmt32 = 0;  // autotune on next use
-        s->fmt_forced = false;
+        s->fmt_forced = s->fmt_default = false;
         return OGSX_OK;
     }
     if (!valid_fmt(s, lanes_per_row))
@@ -2398,6 +2420,7 @@ int ogsx_set_spmv_variant(ogsx_system* s, int lanes_per_row)
     }
     s->fmt64 = s->fmt32 = lanes_per_row;
     s->fmt_forced = true;
+    s->fmt_default = false;
     return OGSX_OK;
 }
 

@@ -177,3 +177,27 @@ def test_noalloc_rows_and_sizes(n, width, method):
     r = b - np.bincount(row, val * xs[0][col], n)
     # the recurrence's residual and the true one differ by rounding
     assert np.linalg.norm(r) <= 1e-11 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("prec", [ox.FP64, ox.FP32_IR])
+@pytest.mark.parametrize("shape", [(9, 7), (70, 60)])
+@pytest.mark.parametrize("bc", [ox.DIRICHLET_ROW, ox.DIRICHLET_SYMMETRIC])
+def test_formats_are_tuned_when_asked_for(shape, prec, bc):
+    """A solve in resident launches times no SpMV format; asking for the
+    formats does, and changes no later solve."""
+    sc = _scenario("quad", shape)
+    system = W.make_system(sc, prec)
+    s = system[1]
+    kw = dict(method=ox.BICGSTAB, dirichlet=bc)
+    first = _solve(sc, system, False, **kw)
+    stands = bc == ox.DIRICHLET_SYMMETRIC  # the diagonal copy, format 25
+    timed = [f for f, _ in s.spmv_tuning()]
+    half = len(timed) // 2 if prec == ox.FP32_IR else len(timed)
+    for part, fmt in ((timed[:half], s.spmv_format()), (timed[half:], s.spmv_format(fp32=True))):
+        if part:
+            assert len(set(part)) == len(part) > 1 and (fmt == 25 if stands else fmt in part)
+    _same(_solve(sc, system, False, **kw), first)
+    _same(_solve(sc, system, True, **kw), first)
+    s.set_spmv_variant(0)
+    _same(_solve(sc, system, False, **kw), first)
+    s.close()
