@@ -264,8 +264,10 @@ struct ogsx_system {
     std::vector<std::pair<int, int>> ev_pending;  // (kind, pool index of start)
     size_t ev_next = 0;
     ProfAcc prof_acc[4];
-    std::vector<void*> allocs;
-    int64_t bytes = 0;  // device bytes allocated
+    std::vector<void*> allocs;    // device blocks
+    char* arena = nullptr;        // unused end of one of them, for small arrays
+    size_t arena_left = 0, arena_next = 0;
+    int64_t bytes = 0;  // device bytes of the arrays
 };
 
 namespace {
@@ -292,17 +294,46 @@ bool use_pool()
     return pool;
 }
 
+// Arrays of less than kArenaOwn share blocks: a release of one array back to
+// the pool costs 11 us, and a system has seventy of them (create, assemble, two
+// solves and destroy on 3,900 rows: 2.95 ms with an allocation per array, 2.11
+// with the blocks).  The first block takes a whole system of up to kArenaFirst;
+// larger systems and later arrays take blocks of kArenaNext, so that little
+// more than one of those is unused.
+constexpr size_t kArenaOwn = size_t(1) << 20, kArenaFirst = size_t(8) << 20,
+                 kArenaNext = size_t(256) << 10, kArenaAlign = 256;
+
+int block_alloc(ogsx_system* s, char** p, size_t bytes)
+{
+    void* q = nullptr;
+    hipError_t e = use_pool() ? hipMallocAsync(&q, bytes, s->stream) : hipMalloc(&q, bytes);
+    if (e != hipSuccess)
+        return fail(OGSX_ENOMEM, std::string("hipMalloc failed: ") + hipGetErrorString(e));
+    s->allocs.push_back(q);
+    *p = (char*)q;
+    return OGSX_OK;
+}
+
 template <typename T>
 int dalloc(ogsx_system* s, T** p, size_t count)
 {
     if (count == 0) count = 1;
-    void* q = nullptr;
-    hipError_t e = use_pool() ? hipMallocAsync(&q, count * sizeof(T), s->stream)
-                              : hipMalloc(&q, count * sizeof(T));
-    if (e != hipSuccess)
-        return fail(OGSX_ENOMEM, std::string("hipMalloc failed: ") + hipGetErrorString(e));
-    s->allocs.push_back(q);
-    s->bytes += (int64_t)(count * sizeof(T));
+    const size_t bytes = count * sizeof(T), room = (bytes + kArenaAlign - 1) & ~(kArenaAlign - 1);
+    char* q = s->arena;
+    if (bytes < kArenaOwn && room <= s->arena_left) {
+        s->arena += room;
+        s->arena_left -= room;
+    } else {
+        const size_t block = bytes < kArenaOwn ? std::max(room, s->arena_next) : bytes;
+        const int rc = block_alloc(s, &q, block);
+        if (rc != OGSX_OK) return rc;
+        if (bytes < kArenaOwn) s->arena_next = kArenaNext;
+        if (block > room && block - room > s->arena_left) {
+            s->arena = q + room;
+            s->arena_left = block - room;
+        }
+    }
+    s->bytes += (int64_t)bytes;
     *p = (T*)q;
     return OGSX_OK;
 }
@@ -1106,6 +1137,8 @@ int ogsx_system_create(const ogsx_pattern* p, int precision, ogsx_system** out)
         return cleanup(fail(OGSX_EHIP, "hipStreamCreate failed"));
     const PatternHost& h = p->h;
     const PatternLayout& Ly = p->L;
+    const size_t total = (size_t)system_bytes(p, precision);
+    s->arena_next = total <= kArenaFirst ? total + (size_t(64) << 10) : kArenaNext;
     if ((rc = dalloc(s, &s->ptr, h.n + 1)) || (rc = dalloc(s, &s->col, h.nnz)) ||
         (rc = dalloc(s, &s->diagpos, h.n)) || (rc = dalloc(s, &s->conn, h.conn.size())) ||
         (rc = dalloc(s, &s->color_elems, h.color_elems.size())) ||
