@@ -2030,13 +2030,18 @@ int ogsx_group_start(ogsx_group* g, ogsx_system* const* systems, int count,
     }
     for (int i : which) OK_TRY(autotune(m->mem[i]));
     share_formats(m, which, g->precision == OGSX_FP32_IR);
+    const bool batched = kmethod != kMethodCgSr;
+    std::vector<int> rest;
     for (int i : which) {
         ogsx_system* s = m->mem[i];
-        OK_TRY(prepare_member(s, cfg, s->stream));
+        int need = 0;
+        OK_TRY(prepare_member(s, cfg, s->stream, batched ? &need : nullptr));
+        rest.push_back(need);
         if (!s->ready) HIP_TRY(hipEventCreateWithFlags(&s->ready, hipEventDisableTiming));
         HIP_TRY(hipEventRecord(s->ready, s->stream));
         HIP_TRY(hipStreamWaitEvent(g->stream, s->ready, 0));
     }
+    if (batched) OK_TRY(prepare_rest(m, which, rest, g->precision == OGSX_FP32_IR));
     return set_start(m, which);
 }
 

@@ -148,6 +148,23 @@ def test_group_of_several_resident_launches(prec):
         system[1].close()
 
 
+@pytest.mark.parametrize("prec", [ox.FP64, ox.FP32_IR])
+@pytest.mark.parametrize("method,bc", [(ox.CG, ox.DIRICHLET_SYMMETRIC), (ox.BICGSTAB, ox.DIRICHLET_ROW)])
+def test_group_members_prepared_together(prec, method, bc):
+    """Members on and off a banded pattern, of several sizes, over two steps
+    (the matrix copies of the first are stale in the second): each member's
+    result is that of its own solves."""
+    scs = [_scenario("line", (1,)), _scenario("quad", (16, 15)), _scenario("quad", (40, 33), permute=True),
+           _scenario("hex", (9, 8, 7)), _scenario("tet", (7, 6, 5), permute=True)]
+    for sc in scs:
+        sc.steps, sc.max_iter = [Step(100.0, 1.0), Step(30.0, 1.0)], 60
+    got = W.run_group(scs, precision=prec, method=method, dirichlet=bc)
+    for sc, x, info in zip(scs, got["x"], got["info"]):
+        system = W.make_system(sc, prec)
+        _same((x, info[-1]), _solve(sc, system, False, method=method, dirichlet=bc))
+        system[1].close()
+
+
 @pytest.mark.parametrize("n,width", [(1, 1), (300, 3), (2048, 9), (2049, 9), (5000, 27), (5000, 29), (262144, 3),
                                      (262145, 3)])
 @pytest.mark.parametrize("method", [ox.CG, ox.BICGSTAB])
