@@ -359,8 +359,9 @@ int ogsx_profile_read(ogsx_system* s, int kind, double* total_ms,
 #define OGSX_PROF_ASSEMBLY 2
 #define OGSX_PROF_VELOCITY 3 /* ogsx_gauss_velocity kernel (on the flow system) */
 /* SpMV storage/launch variant: 0 = autotune (time variants 3, 5, 6, 7, 10,
- * 11, 12, 13, 14, 17, 18, 21, 22, 19, 20 on this matrix at first use and keep the
- * fastest; all of them sum each row in CRS order over rounded products,
+ * 11, 12, 13, 14, 17, 18, 21, 22, 19, 20 on this matrix at the first use that
+ * reads one -- a solve in resident launches or on the diagonal copy reads
+ * none -- and keep the fastest; all of them sum each row in CRS order over rounded products,
  * bit-identical to CSparseMatrix::multiVec, and hand each row to the same
  * thread of the same block, so the dot products the solve fuses into its
  * SpMV round identically too: the choice never changes results; the same
@@ -412,7 +413,8 @@ int ogsx_get_spmv_variant(ogsx_system* s, int* variant);
  * reference (one matrix format there). */
 int ogsx_get_spmv_formats(ogsx_system* s, int* fmt64, int* fmt32);
 /* The autotuner's table: variant and average ms per SpMV launch (FP64 then,
- * for IR systems, FP32 entries); *count = entries available. */
+ * for IR systems, FP32 entries); *count = entries available (0 while a group
+ * solve that reads no tuned format is under way). */
 int ogsx_spmv_tuning(ogsx_system* s, int max_entries, int* variants, double* ms,
                      int* count);
 /* Runs `reps` SpMV launches of the system's FP64 (fp32 = 0) or FP32 matrix
@@ -429,14 +431,15 @@ int ogsx_stream_copy(int64_t bytes, int reps, double* gbs);
 int ogsx_synchronize(ogsx_system* s);
 
 /* ---- persistent launches ---------------------------------------------- */
-/* No counterpart in the reference.  Solves of small systems (and groups of
- * them) spend their time dispatching the dependent launches of each Krylov
- * iteration; a persistent launch runs a batch of iterations in one
+/* No counterpart in the reference.  By default a system that fits the chip
+ * runs a batch of iterations in one resident launch, whose workgroups exchange
+ * their dot products by relaxed atomics; this mode is an older alternative,
+ * in place of those launches: a persistent launch runs a batch of iterations in one
  * cooperative launch of co-resident blocks, with a grid barrier between
  * phases, over the same per-system chunks, so results are bit-identical to
  * the separate launches.  mode: 0 off (default: on MI355X the grid barrier,
- * 12-15 us across the 8 XCDs, costs more than the ~4 us kernel boundary it
- * replaces); 1 auto (running systems of at most 2^19 rows in all, one
+ * 12-15 us across the 8 XCDs with its cache write-backs, costs more than the
+ * ~4 us kernel boundary it replaces); 1 auto (running systems of at most 2^19 rows in all, one
  * slice-based or plain CRS SpMV format, no profiling); 2 whenever the
  * launch shape allows.  Library-wide setting. */
 int ogsx_set_persistent(int mode);

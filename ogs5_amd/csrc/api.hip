@@ -904,6 +904,7 @@ int tune_one(ogsx_system* s, int* fmt_out)
 
 int autotune(ogsx_system* s)
 {
+    if (s->sc.active) return OGSX_OK;  // its vectors are in use
     // what the tuner finds goes where the diagonal copy keeps it, if that
     // stands in for an untimed format
     int* f64 = s->fmt64 == kFmtSymDia ? &s->fmt64_tuned : &s->fmt64;
@@ -2028,7 +2029,8 @@ int ogsx_group_start(ogsx_group* g, ogsx_system* const* systems, int count,
         kmethod = km;
         which.push_back(i);
     }
-    for (int i : which) OK_TRY(autotune(m->mem[i]));
+    for (int i : which)
+        if (reads_tuned_format(m->mem[i], g->precision == OGSX_FP32_IR, kmethod)) OK_TRY(autotune(m->mem[i]));
     share_formats(m, which, g->precision == OGSX_FP32_IR);
     const bool batched = kmethod != kMethodCgSr;
     std::vector<int> rest;
