@@ -577,7 +577,7 @@ def quad_mode(steps_timed=5, cpu=True):
                                "Jacobi-PCG to 1e-10", "dof": sc.n},
         "roofline": None,
         "cpu_baseline": cpu_base,
-        "note": "latency-bound (a few microseconds per kernel, three kernels per CG iteration); "
+        "note": "latency-bound (two exchanges of dot products among workgroups per CG iteration); "
                 "the HBM roofline does not apply at this size",
         "runs": res,
     }))
