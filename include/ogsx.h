@@ -430,6 +430,21 @@ int ogsx_stream_copy(int64_t bytes, int reps, double* gbs);
 /* Synchronises the system's stream. */
 int ogsx_synchronize(ogsx_system* s);
 
+/* ---- resident launches -------------------------------------------------- */
+/* No counterpart in the reference.  A system that fits the chip runs its
+ * Krylov iterations in batches, each one resident launch.  A launch whose
+ * workgroups are not all on the chip within 200 us (other work holds it)
+ * leaves with nothing changed, and the solve goes on in a launch per phase,
+ * trying again after 1, 2 and 4 batches and not after the third time; the
+ * iterates are the same bit for bit.
+ * Counts of the system's batches since its creation, alone and in groups:
+ * *run of them in resident launches, *left of them at such a launch that left. */
+int ogsx_resident_counts(ogsx_system* s, int64_t* run, int64_t* left);
+/* Diagnostic: makes the next `batches` resident launches with this system wait
+ * for one workgroup more than there is, so that they leave as on a taken chip.
+ * (A system of one workgroup waits for nobody and never leaves.) */
+int ogsx_resident_leave(ogsx_system* s, int batches);
+
 /* ---- persistent launches ---------------------------------------------- */
 /* No counterpart in the reference.  By default a system that fits the chip
  * runs a batch of iterations in one resident launch, whose workgroups exchange

@@ -93,6 +93,8 @@ SIGNATURES = {
                                   C.POINTER(C.c_double)]),
     "ogsx_stream_copy": (C.c_int, [_I64, C.c_int, C.POINTER(C.c_double)]),
     "ogsx_synchronize": (C.c_int, [_P]),
+    "ogsx_resident_counts": (C.c_int, [_P, C.POINTER(_I64), C.POINTER(_I64)]),
+    "ogsx_resident_leave": (C.c_int, [_P, C.c_int]),
     "ogsx_set_persistent": (C.c_int, [C.c_int]),
     "ogsx_get_persistent": (C.c_int, [_P, _P]),
     "ogsx_persistent_giveup_probe": (C.c_int, [_P]),
@@ -362,6 +364,18 @@ class System:
         check(lib().ogsx_spmv_tuning(self.h, 32, _ptr(f), _ptr(ms), C.byref(cnt)),
               "ogsx_spmv_tuning")
         return [(int(a), float(b)) for a, b in zip(f[:cnt.value], ms[:cnt.value])]
+
+    def resident_counts(self):
+        """(run, left): batches of iterations that ran in resident launches,
+        and that left one at its census (ogsx_resident_counts)."""
+        run, left = C.c_int64(), C.c_int64()
+        check(lib().ogsx_resident_counts(self.h, C.byref(run), C.byref(left)),
+              "ogsx_resident_counts")
+        return run.value, left.value
+
+    def resident_leave(self, batches: int = 1):
+        """Diagnostic: the next `batches` resident launches leave at their census."""
+        check(lib().ogsx_resident_leave(self.h, int(batches)), "ogsx_resident_leave")
 
     def synchronize(self):
         check(lib().ogsx_synchronize(self.h), "ogsx_synchronize")

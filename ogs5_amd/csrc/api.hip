@@ -217,6 +217,10 @@ struct ogsx_system {
     double* r64 = nullptr;  // IR residual
     double* part = nullptr; // partial sums: 16 x part_stride(G)
     ResSync* rs = nullptr;  // exchange buffers of resident launches
+    // batches in resident launches: run, left at the census, still to be made
+    // to leave (ogsx_resident_leave)
+    int64_t res_run = 0, res_left = 0;
+    int res_leave = 0;
     double* red = nullptr;  // reduced scalars
     KrylovState* st = nullptr;
     // device descriptor of this system and its per-solve parameters
@@ -2429,6 +2433,21 @@ int ogsx_profile_read(ogsx_system* s, int kind, double* total_ms, int64_t* launc
         else
             *bytes_per_launch = 0.0;
     }
+    return OGSX_OK;
+}
+
+int ogsx_resident_counts(ogsx_system* s, int64_t* run, int64_t* left)
+{
+    if (!s) return fail(OGSX_EINVAL, "null system");
+    if (run) *run = s->res_run;
+    if (left) *left = s->res_left;
+    return OGSX_OK;
+}
+
+int ogsx_resident_leave(ogsx_system* s, int batches)
+{
+    if (!s || batches < 0) return fail(OGSX_EINVAL, "bad argument");
+    s->res_leave = batches;
     return OGSX_OK;
 }
 

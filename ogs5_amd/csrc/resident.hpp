@@ -81,7 +81,12 @@ struct ResCensus {
     int pad[14];
 };
 
-// One resident launch: its census entry, workgroups in all and iterations.
+// One resident launch: its census entry, the workgroups to count and
+// iterations.  A launch clears the entry half a ring ahead for a later one, so
+// only launches that take the census may be numbered through the ring: one
+// that does not (k_cg_one, k_bi_one) would leave the entry it skips with an
+// old count and decision, and the launch that takes that entry next would go
+// on, or leave, without counting anyone in.
 struct ResLaunch {
     ResCensus* ring;
     int entry;
