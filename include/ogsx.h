@@ -440,10 +440,16 @@ int ogsx_synchronize(ogsx_system* s);
  * Counts of the system's batches since its creation, alone and in groups:
  * *run of them in resident launches, *left of them at such a launch that left. */
 int ogsx_resident_counts(ogsx_system* s, int64_t* run, int64_t* left);
-/* Diagnostic: makes the next `batches` resident launches with this system wait
- * for one workgroup more than there is, so that they leave as on a taken chip.
- * (A system of one workgroup waits for nobody and never leaves.) */
-int ogsx_resident_leave(ogsx_system* s, int batches);
+/* Diagnostic: makes the next `batches` resident launches with this system fail.
+ * OGSX_RESIDENT_LEAVE: their census waits for one workgroup more than there is,
+ * so they leave as on a taken chip.  OGSX_RESIDENT_EXPIRE: their workgroups wait
+ * for one another for a single poll; a wait that runs out returns OGSX_EHIP from
+ * the solving call, ends the solves of the launch's systems unconverged, with x
+ * undefined, and leaves the systems ready for the next solve.  (A system of one
+ * workgroup waits for nobody and does neither.) */
+#define OGSX_RESIDENT_LEAVE 1
+#define OGSX_RESIDENT_EXPIRE 2
+int ogsx_resident_fail(ogsx_system* s, int how, int batches);
 
 /* ---- persistent launches ---------------------------------------------- */
 /* No counterpart in the reference.  By default a system that fits the chip

@@ -39,6 +39,7 @@ class Elements(C.Structure):
 
 
 IR_RESTART, IR_RELIABLE, IR_RELIABLE_SR = 0, 1, 2
+RESIDENT_LEAVE, RESIDENT_EXPIRE = 1, 2
 
 
 class SolverConfig(C.Structure):
@@ -94,7 +95,7 @@ SIGNATURES = {
     "ogsx_stream_copy": (C.c_int, [_I64, C.c_int, C.POINTER(C.c_double)]),
     "ogsx_synchronize": (C.c_int, [_P]),
     "ogsx_resident_counts": (C.c_int, [_P, C.POINTER(_I64), C.POINTER(_I64)]),
-    "ogsx_resident_leave": (C.c_int, [_P, C.c_int]),
+    "ogsx_resident_fail": (C.c_int, [_P, C.c_int, C.c_int]),
     "ogsx_set_persistent": (C.c_int, [C.c_int]),
     "ogsx_get_persistent": (C.c_int, [_P, _P]),
     "ogsx_persistent_giveup_probe": (C.c_int, [_P]),
@@ -373,9 +374,10 @@ class System:
               "ogsx_resident_counts")
         return run.value, left.value
 
-    def resident_leave(self, batches: int = 1):
-        """Diagnostic: the next `batches` resident launches leave at their census."""
-        check(lib().ogsx_resident_leave(self.h, int(batches)), "ogsx_resident_leave")
+    def resident_fail(self, how: int, batches: int = 1):
+        """Diagnostic: the next `batches` resident launches leave at their census
+        (RESIDENT_LEAVE) or run out of their waits (RESIDENT_EXPIRE)."""
+        check(lib().ogsx_resident_fail(self.h, int(how), int(batches)), "ogsx_resident_fail")
 
     def synchronize(self):
         check(lib().ogsx_synchronize(self.h), "ogsx_synchronize")

@@ -218,9 +218,9 @@ struct ogsx_system {
     double* part = nullptr; // partial sums: 16 x part_stride(G)
     ResSync* rs = nullptr;  // exchange buffers of resident launches
     // batches in resident launches: run, left at the census, still to be made
-    // to leave (ogsx_resident_leave)
+    // to leave or to expire (ogsx_resident_fail)
     int64_t res_run = 0, res_left = 0;
-    int res_leave = 0;
+    int res_leave = 0, res_expire = 0;
     double* red = nullptr;  // reduced scalars
     KrylovState* st = nullptr;
     // device descriptor of this system and its per-solve parameters
@@ -2444,10 +2444,11 @@ int ogsx_resident_counts(ogsx_system* s, int64_t* run, int64_t* left)
     return OGSX_OK;
 }
 
-int ogsx_resident_leave(ogsx_system* s, int batches)
+int ogsx_resident_fail(ogsx_system* s, int how, int batches)
 {
-    if (!s || batches < 0) return fail(OGSX_EINVAL, "bad argument");
-    s->res_leave = batches;
+    if (!s || batches < 0 || (how != OGSX_RESIDENT_LEAVE && how != OGSX_RESIDENT_EXPIRE))
+        return fail(OGSX_EINVAL, "bad argument");
+    (how == OGSX_RESIDENT_LEAVE ? s->res_leave : s->res_expire) = batches;
     return OGSX_OK;
 }
 

@@ -1989,6 +1989,7 @@ __global__ void k_cg_init_final(Grp g, int want)
     st->done = 0;
     st->pend = 0;
     st->resident = 0;
+    st->expired = 0;
     if (P.bnorm_prev > 0.0 && bnorm_new / P.bnorm_prev < P.tol) {
         st->error = bnorm_new / P.bnorm_prev;
         st->bnorm = bnorm_new;
@@ -2393,6 +2394,7 @@ __global__ void k_bi_init_final(Grp g, int want)
     st->done = 0;
     st->pend = 0;
     st->resident = 0;
+    st->expired = 0;
     st->rho0 = 1.0;
     st->alpha = 1.0;
     st->omega = 1.0;

@@ -103,9 +103,10 @@ struct KrylovState {
     double sr_alp;    // alpha of the last update
     int sr_it;        // iterations completed (>= iter)
     int resident;     // last resident launch: 0 ran, 1 left at its census
-                      // (nothing done), 2 a wait ran out (resident.hpp)
+                      // (nothing done)
     int row_max;      // longest row (zero-allocation solve only)
-    int pad;
+    int expired;      // a workgroup's wait in a resident launch ran out: the
+                      // vectors are of no one iteration (resident.hpp)
 };
 
 }  // namespace ogsx

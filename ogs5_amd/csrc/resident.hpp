@@ -92,6 +92,7 @@ struct ResLaunch {
     int entry;
     int wgs;
     int iters;
+    unsigned polls = kResPolls;  // of one wait
 };
 
 template <typename T>
@@ -126,6 +127,27 @@ __global__ __launch_bounds__(kBlock) void k_res_clear(ResSync* rs, size_t count)
          i += (size_t)gridDim.x * kBlock)
         rs->slot[i] = kSlotEmpty;
     if (blockIdx.x == 0 && threadIdx.x == 0) rs->phase = 0;
+}
+
+// After a wait that ran out: empties the exchange buffers, whose slots and
+// phase the workgroups no longer agree on, and stops the solve, so that no later
+// launch goes on from its vectors.
+__global__ __launch_bounds__(kBlock) void k_res_stop(const SysDev* sys)
+{
+    const size_t count = res_slot_count(sys->G);
+    for (size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x; i < count;
+         i += (size_t)gridDim.x * kBlock)
+        sys->rs->slot[i] = kSlotEmpty;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        sys->rs->phase = 0;
+        sys->st->done = 4;
+        sys->st->pend = 0;
+        sys->st->expired = 0;
+        if (sys->irs) {
+            sys->irs->status = 0;
+            sys->irs->action = 0;
+        }
+    }
 }
 
 // Counts the launch's workgroups in; true when all of them are resident.  A
@@ -178,6 +200,7 @@ struct ResExchange {
     double (*sw)[4 * VB];  // [kSlotVals] wave sums
     double (*sm)[4];       // [kSlotVals] sums of the waves that poll
     int* ok;
+    unsigned limit;        // polls of one wait
 
     __device__ __forceinline__ OGSX_GL unsigned long long* at(int s, int k, int copy) const
     {
@@ -252,7 +275,7 @@ struct ResExchange {
                     for (int k = 0; k < NV; k++) got[k] = agent_load(at(set, k, w % kSlotCopies) + t);
 #pragma unroll
                     for (int k = 0; k < NV; k++) wait = wait || got[k] == kSlotEmpty;
-                    if (wait && ++polls > kResPolls) {
+                    if (wait && ++polls > limit) {
                         *ok = 0;
                         break;
                     }
@@ -425,7 +448,7 @@ __global__ __launch_bounds__(kBlock * VB) void k_cg_resident(Grp g, ResLaunch L)
     double ir_error = 0.0, maxr = 0.0;
     double rr = st->rr;
     ResExchange<VB> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, G / VB,
-                       sw, sm, &ok};
+                       sw, sm, &ok, L.polls};
     if (tid == 0) ok = 1;
     if (!res_census(L, idle, &flag)) {
         if (!idle && w == 0 && tid == 0) st->resident = 1;
@@ -538,6 +561,8 @@ __global__ __launch_bounds__(kBlock * VB) void k_cg_resident(Grp g, ResLaunch L)
         v.r[row] = r;
         v.p[row] = p;
     }
+    // (by any workgroup: the others may have had their sums and gone on)
+    if (!good && tid == 0) agent_store(&st->expired, 1);
     if (w == 0 && tid == 0) {
         st->error = error;
         st->rr = rr;
@@ -545,7 +570,7 @@ __global__ __launch_bounds__(kBlock * VB) void k_cg_resident(Grp g, ResLaunch L)
         st->alpha = alpha_d;
         st->iter = it;
         st->done = done;
-        st->resident = good ? 0 : 2;
+        st->resident = 0;
         S.rs->phase = ex.set;
         if (IR && updates > 0) {
             OGSX_GL IRState* R = gl(S.irs);
@@ -592,7 +617,7 @@ __global__ __launch_bounds__(kBlock * VB) void k_bi_resident(Grp g, ResLaunch L)
     double rho0 = st->rho0, rho1 = st->rho1, alpha_d = st->alpha, omega_d = st->omega;
     double error = st->error;
     ResExchange<VB> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, G / VB,
-                       sw, sm, &ok};
+                       sw, sm, &ok, L.polls};
     if (tid == 0) ok = 1;
     if (!res_census(L, idle, &flag)) {
         if (!idle && w == 0 && tid == 0) st->resident = 1;
@@ -717,6 +742,8 @@ __global__ __launch_bounds__(kBlock * VB) void k_bi_resident(Grp g, ResLaunch L)
             part[k * part_stride(G) + kBlock * (c % q) + c / q] =
                 ((sw[k][4 * vb] + sw[k][4 * vb + 1]) + sw[k][4 * vb + 2]) + sw[k][4 * vb + 3];
     }
+    // (by any workgroup: the others may have had their sums and gone on)
+    if (!good && tid == 0) agent_store(&st->expired, 1);
     if (w == 0 && tid == 0) {
         st->error = error;
         st->rho0 = rho0;
@@ -726,7 +753,7 @@ __global__ __launch_bounds__(kBlock * VB) void k_bi_resident(Grp g, ResLaunch L)
         st->iter = it;
         st->pend = pend;
         st->done = done;
-        st->resident = good ? 0 : 2;
+        st->resident = 0;
         S.rs->phase = ex.set;
     }
 }
@@ -1241,7 +1268,7 @@ __global__ __launch_bounds__(kBlock * kStreamVb) void k_cg_stream(Grp g, ResLaun
     const double bnorm = st->bnorm;
     const double tol = gl(S.prm)->tol, upd_thresh = gl(S.prm)->upd_thresh;
     double rr = st->rr;
-    ResExchange<VB> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, nwg, sw, sm, &ok};
+    ResExchange<VB> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, nwg, sw, sm, &ok, L.polls};
     if (tid == 0) ok = 1;
     if (!res_census(L, idle, &flag)) {
         if (!idle && w == 0 && tid == 0) st->resident = 1;
@@ -1377,6 +1404,8 @@ __global__ __launch_bounds__(kBlock * kStreamVb) void k_cg_stream(Grp g, ResLaun
             out.p[i] = agent_load(src + i);
         if constexpr (XL) out.x[i] = xl[at(i)];
     }
+    // (by any workgroup: the others may have had their sums and gone on)
+    if (!good && tid == 0) agent_store(&st->expired, 1);
     if (w == 0 && tid == 0) {
         st->error = error;
         st->rr = rr;
@@ -1384,7 +1413,7 @@ __global__ __launch_bounds__(kBlock * kStreamVb) void k_cg_stream(Grp g, ResLaun
         st->alpha = alpha_d;
         st->iter = it;
         st->done = done;
-        st->resident = good ? 0 : 2;
+        st->resident = 0;
         S.rs->phase = ex.set;
     }
 }
@@ -1460,7 +1489,7 @@ __global__ __launch_bounds__(kBlock * kStreamVb) void k_bi_stream(Grp g, ResLaun
     const double tol = gl(S.prm)->tol;
     double rho0 = st->rho0, rho1 = st->rho1, alpha_d = st->alpha, omega_d = st->omega;
     double error = st->error;
-    ResExchange<VB> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, nwg, sw, sm, &ok};
+    ResExchange<VB> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, nwg, sw, sm, &ok, L.polls};
     if (tid == 0) ok = 1;
     if (!res_census(L, idle, &flag)) {
         if (!idle && w == 0 && tid == 0) st->resident = 1;
@@ -1652,6 +1681,8 @@ __global__ __launch_bounds__(kBlock * kStreamVb) void k_bi_stream(Grp g, ResLaun
             part[k * part_stride(G) + kBlock * (c % q) + c / q] =
                 ((sw[k][4 * vb] + sw[k][4 * vb + 1]) + sw[k][4 * vb + 2]) + sw[k][4 * vb + 3];
     }
+    // (by any workgroup: the others may have had their sums and gone on)
+    if (!good && tid == 0) agent_store(&st->expired, 1);
     if (w == 0 && tid == 0) {
         st->error = error;
         st->rho0 = rho0;
@@ -1661,7 +1692,7 @@ __global__ __launch_bounds__(kBlock * kStreamVb) void k_bi_stream(Grp g, ResLaun
         st->iter = it;
         st->pend = pend;
         st->done = done;
-        st->resident = good ? 0 : 2;
+        st->resident = 0;
         S.rs->phase = ex.set;
     }
 }

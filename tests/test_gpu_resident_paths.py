@@ -8,7 +8,7 @@ import pytest
 import ogs5_amd as ox
 from ogs5_amd import workloads as W
 
-from test_gpu_resident import _scenario, _solve
+from test_gpu_resident import _same, _scenario, _solve
 
 pytestmark = pytest.mark.gpu
 
@@ -23,7 +23,7 @@ def test_one_workgroup_launches_keep_out_of_the_census_ring():
     sc = _scenario("quad", (40, 40))  # CG: one workgroup; BiCGStab: several
     system = W.make_system(sc, ox.FP64)
     s = system[1]
-    s.resident_leave(1)
+    s.resident_fail(ox.RESIDENT_LEAVE)
     _solve(sc, system, False, method=ox.BICGSTAB)
     assert s.resident_counts()[1] == 1
     for _ in range(40):
@@ -33,3 +33,80 @@ def test_one_workgroup_launches_keep_out_of_the_census_ring():
         _solve(sc, system, False, method=ox.BICGSTAB)
     assert s.resident_counts() == (run + 80, 1)
     s.close()
+
+
+# (kind, shape, method, elimination): a thread per row, and the streamed matrix
+SEVERAL = [("quad", (200, 199), ox.CG, ox.DIRICHLET_SYMMETRIC),
+           ("quad", (150, 140), ox.BICGSTAB, ox.DIRICHLET_ROW),
+           ("hex", (65, 64, 63), ox.CG, ox.DIRICHLET_SYMMETRIC),
+           ("tet", (66, 64, 62), ox.BICGSTAB, ox.DIRICHLET_ROW)]
+
+
+@pytest.mark.parametrize("prec", [ox.FP64, ox.FP32_IR])
+@pytest.mark.parametrize("kind,shape,method,bc", SEVERAL)
+def test_an_expired_wait_ends_the_solve(kind, shape, method, bc, prec):
+    """Workgroups that give up waiting at once (every one of them still runs to
+    its end): the call fails, the solve is over and unconverged, and the next one
+    finds nothing of it."""
+    sc = _scenario(kind, shape)
+    kw = dict(method=method, dirichlet=bc)
+    system = W.make_system(sc, prec)
+    s = system[1]
+    ref = _solve(sc, system, True, **kw)
+    s.resident_fail(ox.RESIDENT_EXPIRE)
+    with pytest.raises(ox.OgsxError, match="too long"):
+        _solve(sc, system, False, **kw)
+    active, info = ox.solve_status(s)
+    assert not active and info["converged"] == 0 and info["ret"] == 0
+    run = s.resident_counts()[0]
+    _same(_solve(sc, system, False, **kw), ref)
+    assert s.resident_counts()[0] > run
+    s.close()
+
+
+def test_an_expired_wait_in_a_group():
+    """The launch of the two quads expires: both are over, and the hexes, in a
+    launch of their own, go on to the result they have alone.  Then the whole
+    group again."""
+    scs = [_scenario("quad", (90, 80)), _scenario("quad", (101, 70)), _scenario("hex", (22, 20, 18))]
+    refs = []
+    for sc in scs:
+        system = W.make_system(sc, ox.FP64)
+        refs.append(_solve(sc, system, True))
+        system[1].close()
+    systems = [W.make_system(sc, ox.FP64) for sc in scs]
+    mem = [s for _, s in systems]
+    g = ox.Group(ox.FP64)
+    for s in mem:
+        g.add(s)
+
+    def start():
+        for sc, s in zip(scs, mem):
+            s.set_vector(ox.VEC_UOLD, sc.u0)
+            s.set_vector(ox.VEC_X, sc.u0)
+            s.initialize()
+            s.assemble(sc.steps[0].dt, sc.steps[0].theta)
+            s.set_dirichlet(sc.bc_idx, sc.bc_val, ox.DIRICHLET_SYMMETRIC)
+        g.start(mem, method=ox.CG, tol=scs[0].tol, max_iter=40)
+
+    def check(k):
+        active, info = ox.solve_status(mem[k])
+        assert not active
+        _same((mem[k].get_vector(ox.VEC_X), info), refs[k])
+
+    start()
+    mem[0].resident_fail(ox.RESIDENT_EXPIRE)
+    with pytest.raises(ox.OgsxError, match="too long"):
+        g.advance(10)
+    for s in mem[:2]:
+        active, info = ox.solve_status(s)
+        assert not active and info["converged"] == 0
+    assert g.advance(1000) == 0
+    check(2)
+    start()
+    assert g.advance(1000) == 0
+    for k in range(3):
+        check(k)
+    g.close()
+    for s in mem:
+        s.close()
