@@ -110,3 +110,100 @@ def test_an_expired_wait_in_a_group():
     g.close()
     for s in mem:
         s.close()
+
+
+@pytest.mark.parametrize("prec", [ox.FP64, ox.FP32_IR])
+@pytest.mark.parametrize("leaves", [1, 2, 3])
+@pytest.mark.parametrize("kind,shape,method,bc", SEVERAL)
+def test_solve_goes_on_where_a_launch_left(kind, shape, method, bc, leaves, prec):
+    """Launches that leave (as when other work holds the chip): the solve goes on
+    in separate launches, tries again, and after the third time no more; the
+    iterates stay those of separate launches."""
+    sc = _scenario(kind, shape)
+    sc.max_iter = 3000
+    kw = dict(method=method, dirichlet=bc)
+    system = W.make_system(sc, prec)
+    s = system[1]
+    ref = _solve(sc, system, True, **kw)
+    assert s.resident_counts() == (0, 0)
+    s.resident_fail(ox.RESIDENT_LEAVE, leaves)
+    _same(_solve(sc, system, False, **kw), ref)
+    run, left = s.resident_counts()
+    # (a solve of a few batches may end before its next try)
+    assert 1 <= left <= leaves and (left < 3 or run == 0)
+    s.resident_fail(ox.RESIDENT_LEAVE, 0)
+    _same(_solve(sc, system, False, **kw), ref)
+    assert s.resident_counts()[0] > run and s.resident_counts()[1] == left
+    s.close()
+
+
+@pytest.mark.parametrize("prec", [ox.FP64, ox.FP32_IR])
+@pytest.mark.parametrize("kind,shape,method,bc", SEVERAL)
+def test_resident_and_separate_launches_by_turns(kind, shape, method, bc, prec):
+    """A launch that leaves between two that run, by small budgets of a group of
+    one: resident, separate and resident iterations of one solve."""
+    sc = _scenario(kind, shape)
+    kw = dict(method=method, dirichlet=bc)
+    system = W.make_system(sc, prec)
+    ref = _solve(sc, system, True, **kw)
+    s = system[1]
+    s.set_vector(ox.VEC_UOLD, sc.u0)
+    s.set_vector(ox.VEC_X, sc.u0)
+    W._prepare_step(sc, s, 0, bc, False)
+    g = ox.Group(prec)
+    g.add(s)
+    g.start([s], method=method, tol=sc.tol, max_iter=sc.max_iter)
+    seen = []
+    for budget, leave in ((5, 0), (7, 1), (3, 0), (6, 1)):
+        before = s.resident_counts()
+        s.resident_fail(ox.RESIDENT_LEAVE, leave)
+        g.advance(budget)
+        seen.append(tuple(b - a for a, b in zip(before, s.resident_counts())))
+        if not ox.solve_status(s)[0]:
+            break
+    while g.advance(1000):
+        pass
+    # run; left; separate (the wait after a leave); run again or left
+    assert seen[0] == (1, 0) and (0, 1) in seen
+    _same((s.get_vector(ox.VEC_X), ox.solve_status(s)[1]), ref)
+    g.close()
+    s.close()
+
+
+def _star(leaves):
+    """Line elements from one node: its row has leaves + 1 entries."""
+    from ogs5_amd.mesh import LINE2, Mesh
+    z = np.zeros(leaves + 1)
+    x = np.concatenate([[0.0], 1.0 + np.arange(leaves) / leaves])
+    conn = np.stack([np.zeros(leaves, np.int64), np.arange(1, leaves + 1)], 1)
+    sc = _scenario("line", (leaves,))
+    sc.mesh = Mesh(LINE2, 1, x, z, z.copy(), conn, (leaves,), (1.0,), np.arange(leaves))
+    sc.bc_idx, sc.bc_val = np.array([0]), np.array([1.0])
+    return sc
+
+
+# longest rows and most rows of each kind of launch, and one past them
+@pytest.mark.parametrize("prec", [ox.FP64, ox.FP32_IR])
+@pytest.mark.parametrize("make,method,fits", [
+    (lambda: _star(26), ox.CG, True), (lambda: _star(27), ox.CG, False),
+    # (past 27 entries BiCGStab streams a matrix with a stencil dictionary)
+    (lambda: _star(26), ox.BICGSTAB, True), (lambda: _star(27), ox.BICGSTAB, True),
+    (lambda: _scenario("quad", (511, 511), permute=True), ox.CG, True),
+    (lambda: _scenario("quad", (512, 511), permute=True), ox.CG, False),
+    (lambda: _scenario("quad", (512, 511)), ox.CG, True),
+    (lambda: _scenario("quad", (361, 361), permute=True), ox.BICGSTAB, True),
+    (lambda: _scenario("quad", (361, 362), permute=True), ox.BICGSTAB, False),
+    (lambda: _scenario("quad", (361, 362)), ox.BICGSTAB, True)])
+def test_sizes_that_run_resident(make, method, fits, prec):
+    """... and profiling, which keeps a solve to separate launches."""
+    sc = make()
+    sc.max_iter = 12
+    kw = dict(method=method, dirichlet=ox.DIRICHLET_ROW if method == ox.BICGSTAB
+              else ox.DIRICHLET_SYMMETRIC)
+    system = W.make_system(sc, prec)
+    s = system[1]
+    ref = _solve(sc, system, True, **kw)
+    assert s.resident_counts() == (0, 0)
+    _same(_solve(sc, system, False, **kw), ref)
+    assert (s.resident_counts()[0] > 0) == fits and s.resident_counts()[1] == 0
+    s.close()
