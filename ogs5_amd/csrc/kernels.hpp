@@ -812,6 +812,15 @@ __device__ __forceinline__ void spmv_sell_x2(const GMat<VT>& m, const OGSX_GL XT
     }
 }
 
+// LDS written by some lanes of a wavefront and read by others of the same
+// wavefront: the wavefront's LDS accesses complete in order once waited for.
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Plain CRS with one thread per row: each row summed left to right over
 // rounded products (CSparseMatrix::multiVec's order,
 // FEM/matrix_class.cpp:1527-1538).  Needs no layout beyond ptr, col and
@@ -821,18 +830,65 @@ __device__ __forceinline__ void spmv_sell_x2(const GMat<VT>& m, const OGSX_GL XT
 // slices, thread t the rows R0 + t + 256 j -- so the fused dot products of
 // the solve kernels (accumulated per thread in that order, then reduced in
 // a fixed tree) round exactly as with every SELL-64 format.
+//
+// A wave takes the entries of its 64 rows kCrsTile at a time, neighbouring
+// lanes neighbouring entries, and hands the products to the rows' threads
+// through LDS.  (Each thread reading its own row leaves the lanes a row's
+// length apart: every line of the matrix is then loaded once per entry in it,
+// from the L1 only while the waves' 64 rows of lines fit there -- 27-entry rows
+// do for four waves on a compute unit, not for sixteen.  Zero-allocation CG, us
+// per iteration: 227,000 rows of 27 entries 33, read by row 211; 439,000 44 and
+// 372; 91,000 rows of 16 19 and 27; 361,000 of 9 27 and 35; 300,000 of 3, where
+// most of a tile is empty, 19.3 and 18.9.)  The last tile of a slice takes half
+// as many loads where that is enough: fewer for every entry it has is slower
+// (each load behind a branch: 227,000 rows 36 us).
+constexpr int kCrsU = 8;                  // entries per lane at a time
+constexpr int kCrsTile = 64 * kCrsU;
 template <typename VT, typename XT, typename ACC, typename Epi>
 __device__ __forceinline__ void spmv_crs1(const GMat<VT>& m, const OGSX_GL XT* __restrict__ x,
                                           int G, int b, Epi&& epi)
 {
 #pragma clang fp contract(off)
+    __shared__ ACC stage[kBlock / 64][kCrsTile];
     int beg, end;
     row_chunk(m.n, G, b, beg, end);
-    for (int r = beg + chunk_thread(); r < end; r += kBlock) {
-        const int k1 = m.ptr[r + 1];
+    const int lane = chunk_thread() & 63, wave = chunk_thread() >> 6;
+    ACC* const st = stage[wave];
+    for (int r0 = beg + 64 * wave; r0 < end; r0 += kBlock) {
+        const int r = min(r0 + lane, end - 1);
+        const bool have = r0 + lane < end;
+        const int k0 = m.ptr[r], k1 = have ? m.ptr[r + 1] : k0;
+        const int first = __builtin_amdgcn_readfirstlane(m.ptr[r0]);
+        const int count = __builtin_amdgcn_readfirstlane(m.ptr[min(r0 + 64, end)]) - first;
         ACC s = 0;
-        for (int k = m.ptr[r]; k < k1; k++) s += (ACC)m.val[k] * (ACC)x[m.col[k]];
-        epi(r, s);
+        for (int t0 = 0; t0 < count;) {
+            const int left = count - t0;  // (t0 + kCrsTile may not be an int)
+            const auto take = [&](auto slots) {
+                constexpr int U = decltype(slots)::value;
+                VT a[U];
+                int c[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int k = first + t0 + min(64 * u + lane, left - 1);
+                    a[u] = m.val[k];
+                    c[u] = m.col[k];
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) st[64 * u + lane] = (ACC)a[u] * (ACC)x[c[u]];
+            };
+            if (left > kCrsTile / 2)
+                take(std::integral_constant<int, kCrsU>{});
+            else
+                take(std::integral_constant<int, kCrsU / 2>{});
+            wave_lds_sync();
+            const int e0 = max(k0 - first - t0, 0), e1 = min(k1 - first - t0, kCrsTile);
+#pragma unroll 4
+            for (int e = e0; e < e1; e++) s = s + st[e];
+            wave_lds_sync();
+            if (left <= kCrsTile) break;
+            t0 += kCrsTile;
+        }
+        if (have) epi(r, s);
     }
 }
 
@@ -1435,15 +1491,6 @@ __device__ __forceinline__ int loc_match(uint64_t w, int c)
 #pragma unroll
     for (int j = 0; j < NPE; j++) jm = (int)((w >> (8 * j)) & 0xff) == c ? j : jm;
     return jm;
-}
-
-// LDS written by some lanes of a wavefront and read by others of the same
-// wavefront: the wavefront's LDS accesses complete in order once waited for.
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // The row's records are taken G at a time: lane t loads record t of the
