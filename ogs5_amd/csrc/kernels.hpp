@@ -162,20 +162,37 @@ struct PartialLoads {
 // that the reduction can wait for the partials (from L2) while the rows
 // (from HBM) are still in flight: a wait on the memory counter covers every
 // load issued before the one awaited.
-template <int NV>
+//
+// FEW: only the q = 1, 2 or 4 loads that systems of up to kStreamMaxRows rows
+// have: with a block to every 256 rows each load past those was as much work
+// again in every block (160,000 rows, BiCGStab on the diagonal copy: with the
+// rows' own of batch_slots 30.0 -> 25.7 us per iteration).  The kernels of the
+// largest systems take all eight in one go: 1 % faster there than by the branch.
+template <int NV, bool FEW = true>
 __device__ __forceinline__ void load_partials(const OGSX_GL double* partials, int G,
                                               PartialLoads<NV>& P)
 {
-    const int q = part_q(G), t = threadIdx.x;
+    const int q = __builtin_amdgcn_readfirstlane(part_q(G)), t = threadIdx.x;
+    const auto take = [&](auto slots) {
+        constexpr int U = decltype(slots)::value;
 #pragma unroll
-    for (int k = 0; k < NV; k++)
+        for (int k = 0; k < NV; k++)
 #pragma unroll
-        for (int j = 0; j < kPartialBatch; j++) {
-            // clamped index: every load is issued unpredicated
-            const bool have = j < q && q * t + j < G;
-            const double x = partials[k * part_stride(G) + (have ? kBlock * j + t : 0)];
-            P.t[k][j] = have ? x : 0.0;
-        }
+            for (int j = 0; j < kPartialBatch; j++) {
+                P.t[k][j] = 0.0;
+                if (j >= U) continue;
+                // clamped index: every load is issued unpredicated
+                const bool have = j < q && q * t + j < G;
+                const double x = partials[k * part_stride(G) + (have ? kBlock * j + t : 0)];
+                P.t[k][j] = have ? x : 0.0;
+            }
+    };
+    if (FEW && q <= 2)
+        take(std::integral_constant<int, 2>{});
+    else if (FEW && q == 4)
+        take(std::integral_constant<int, 4>{});
+    else
+        take(std::integral_constant<int, kPartialBatch>{});
 }
 
 // Completes reduce_partials from loads made by load_partials.
@@ -263,8 +280,8 @@ __device__ __forceinline__ void vec_chunk(int n, int G, int b, Body&& body)
 }
 
 // The rows of chunk b, kVecU per thread at a time: load(k, u) reads row k
-// into slot u for all kVecU slots (rows past the chunk's end read its last
-// row and are not used), then apply(k, u) runs for the slots inside the
+// into slot u for all kVecU slots (or those the chunk has at all, see
+// batch_slots; rows past its end read its last row and are not used), then apply(k, u) runs for the slots inside the
 // chunk, in ascending row order.  A thread thus waits for memory once per
 // batch instead of once (or, where stores may alias the next row's loads,
 // several times) per row; per-thread order, hence every sum, is that of
@@ -274,6 +291,20 @@ __device__ __forceinline__ void vec_chunk(int n, int G, int b, Body&& body)
 // returns false the rows are left alone.
 constexpr int kVecU = 4;
 
+// The slots of that batch which a chunk of `rows` rows has at all (the same for
+// the block): f of 1, 2 or kVecU of them.
+template <typename F>
+__device__ __forceinline__ void batch_slots(int rows, F&& f)
+{
+    const int r = __builtin_amdgcn_readfirstlane(rows);
+    if (r <= kBlock)
+        f(std::integral_constant<int, 1>{});
+    else if (r <= 2 * kBlock)
+        f(std::integral_constant<int, 2>{});
+    else
+        f(std::integral_constant<int, kVecU>{});
+}
+
 template <typename Load, typename Mid, typename Apply>
 __device__ __forceinline__ bool vec_chunk_batched_mid(int n, int G, int b, Load&& load, Mid&& mid,
                                                       Apply&& apply)
@@ -282,10 +313,11 @@ __device__ __forceinline__ bool vec_chunk_batched_mid(int n, int G, int b, Load&
     row_chunk(n, G, b, beg, end);
     const int last = end - 1;
     int i = beg + threadIdx.x;
-    if (i < end) {
+    if (i < end)
+        batch_slots(end - beg, [&](auto slots) {
 #pragma unroll
-        for (int u = 0; u < kVecU; u++) load(min(i + u * kBlock, last), u);
-    }
+            for (int u = 0; u < decltype(slots)::value; u++) load(min(i + u * kBlock, last), u);
+        });
     if (!mid()) return false;
     for (bool loaded = true; i < end; i += kVecU * kBlock, loaded = false) {
         if (!loaded) {
@@ -2092,10 +2124,11 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv(Grp g)
 // ms).  Where matrix and vectors fit, cached streams are faster.
 //
 // SMALL: a member of the launch has chunks of fewer than U kBlock rows
-// (systems of up to 262,144 rows), whose threads would otherwise take their
+// (systems of up to 1.05 million rows), whose threads would otherwise take their
 // 1-3 rows one memory round trip at a time.  Such a chunk's rows are then
 // loaded as one batch, before the partials are reduced, with indices past
-// the chunk clamped to its last row (loaded, not used).  Rows are updated
+// the chunk clamped to its last row (loaded, not used; batch_slots leaves out
+// the loads no row of the chunk needs).  Rows are updated
 // and summed in the same order either way, so both forms give the same
 // bits; the host picks SMALL only when some running member needs it (the
 // 256-instance ensemble: 5-7 % faster; on 128^3 hexes the SMALL form ran
@@ -2122,7 +2155,7 @@ __device__ __forceinline__ void cg_update_body(const Grp& g, int vb)
     // issued before the partials are reduced, so their latency overlaps
     // partials first, then the first batch of rows (see load_partials)
     PartialLoads<1> pl;
-    load_partials<1>(gl(S.part), c.G, pl);
+    load_partials<1, SMALL>(gl(S.part), c.G, pl);
     T xi[U], pi[U], ri[U], si[U], di[U];
     const bool first = i + (U - 1) * kBlock < end;
     // a chunk of one full batch plus fewer than kBlock rows (1024-1280
@@ -2149,15 +2182,17 @@ __device__ __forceinline__ void cg_update_body(const Grp& g, int vb)
             dt = ld<VNT>(d + k);
         }
     } else if (SMALL && i < end) {
+        batch_slots(end - beg, [&](auto slots) {
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int k = min(i + u * kBlock, end - 1);
-            xi[u] = ld<VNT>(x + k);
-            pi[u] = ld<VNT>(p + k);
-            ri[u] = ld<VNT>(r + k);
-            si[u] = ld<VNT>(sv + k);
-            di[u] = ld<VNT>(d + k);
-        }
+            for (int u = 0; u < decltype(slots)::value; u++) {
+                const int k = min(i + u * kBlock, end - 1);
+                xi[u] = ld<VNT>(x + k);
+                pi[u] = ld<VNT>(p + k);
+                ri[u] = ld<VNT>(r + k);
+                si[u] = ld<VNT>(sv + k);
+                di[u] = ld<VNT>(d + k);
+            }
+        });
     }
     double ps[1];
     finish_partials<1>(gl(S.part), c.G, pl, ps);
@@ -2255,7 +2290,7 @@ __device__ __forceinline__ void cg_direction_body(const Grp& g, int vb)
     int i = beg + threadIdx.x;
     // first batch loaded before the reduction (independent of beta)
     PartialLoads<2> pl;  // partials first, then the first batch of rows
-    load_partials<2>(gl(S.part) + 4 * part_stride(c.G), c.G, pl);
+    load_partials<2, SMALL>(gl(S.part) + 4 * part_stride(c.G), c.G, pl);
     T pi[U], ri[U], di[U];
     const bool first = i + (U - 1) * kBlock < end;
     // the extra row of a chunk of 1024-1280 rows, as in the update
@@ -2276,13 +2311,15 @@ __device__ __forceinline__ void cg_direction_body(const Grp& g, int vb)
             dt = ld<VNT>(d + k);
         }
     } else if (SMALL && i < end) {  // a chunk's one, partial batch (as in the update)
+        batch_slots(end - beg, [&](auto slots) {
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int k = min(i + u * kBlock, end - 1);
-            pi[u] = ld<VNT>(p + k);
-            ri[u] = ld<VNT>(r + k);
-            di[u] = ld<VNT>(d + k);
-        }
+            for (int u = 0; u < decltype(slots)::value; u++) {
+                const int k = min(i + u * kBlock, end - 1);
+                pi[u] = ld<VNT>(p + k);
+                ri[u] = ld<VNT>(r + k);
+                di[u] = ld<VNT>(d + k);
+            }
+        });
     }
     double s[2];
     finish_partials<2>(gl(S.part) + 4 * part_stride(c.G), c.G, pl, s);
