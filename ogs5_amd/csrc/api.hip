@@ -1940,6 +1940,36 @@ void share_formats(MemberSet* m, const std::vector<int>& which, bool ir)
         }
     }
 }
+
+// Starting systems that read no tuned format (untimed_format) take one that the
+// others' solves read, where they can, so that the two can share launches
+// (join_rest).  The choice never changes a result.
+void borrow_formats(MemberSet* m, const std::vector<int>& which, bool ir, int kmethod)
+{
+    for (int slot = 0; slot < (ir ? 2 : 1); slot++) {
+        std::vector<int> inuse;
+        auto tuned = [&](ogsx_system* s) {
+            const int f = slot == 0 ? s->fmt64 : s->fmt32;
+            if (f != 0 && f != kFmtSymDia && !s->fmt_default) inuse.push_back(f);
+        };
+        for (ogsx_system* s : m->mem)
+            if (s->sc.active) tuned(s);
+        for (int i : which) tuned(m->mem[i]);
+        for (int i : which) {
+            ogsx_system* s = m->mem[i];
+            if (reads_tuned_format(s, ir, kmethod) || (s->dia_ok && s->a_symmetric)) continue;
+            int& f = slot == 0 ? (s->fmt64 == kFmtSymDia ? s->fmt64_tuned : s->fmt64)
+                               : (s->fmt32 == kFmtSymDia ? s->fmt32_tuned : s->fmt32);
+            if (f != 0 && !s->fmt_default) continue;
+            untimed_format(s);
+            for (int u : inuse)
+                if (valid_fmt(s, u) && (!needs_extra_layouts(u) || s->sell_c32)) {
+                    f = u;
+                    break;
+                }
+        }
+    }
+}
 }  // namespace
 
 extern "C" {
@@ -2036,6 +2066,7 @@ int ogsx_group_start(ogsx_group* g, ogsx_system* const* systems, int count,
     for (int i : which)
         if (reads_tuned_format(m->mem[i], g->precision == OGSX_FP32_IR, kmethod)) OK_TRY(autotune(m->mem[i]));
     share_formats(m, which, g->precision == OGSX_FP32_IR);
+    borrow_formats(m, which, g->precision == OGSX_FP32_IR, kmethod);
     const bool batched = kmethod != kMethodCgSr;
     std::vector<int> rest;
     for (int i : which) {

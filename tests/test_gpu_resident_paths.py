@@ -207,3 +207,42 @@ def test_sizes_that_run_resident(make, method, fits, prec):
     _same(_solve(sc, system, False, **kw), ref)
     assert (s.resident_counts()[0] > 0) == fits and s.resident_counts()[1] == 0
     s.close()
+
+
+@pytest.mark.parametrize("prec", [ox.FP64, ox.FP32_IR])
+@pytest.mark.parametrize("method,bc", [(ox.CG, ox.DIRICHLET_SYMMETRIC), (ox.BICGSTAB, ox.DIRICHLET_ROW)])
+@pytest.mark.parametrize("fmt,joins", [(5, True), (9, True), (0, False)])
+def test_small_members_join_separate_launches(method, bc, prec, fmt, joins):
+    """A group where one member has a format set, and so separate launches: the
+    small others go along in them, in its format, and take resident ones once it
+    is done; where none does, all are resident."""
+    scs = [_scenario("quad", (31, 30), seed=1), _scenario("quad", (40, 33), permute=True),
+           _scenario("quad", (52, 47), permute=True)]
+    refs, mem = [], []
+    for sc in scs:
+        sc.max_iter = 30
+        system = W.make_system(sc, prec)
+        refs.append(_solve(sc, system, True, method=method, dirichlet=bc))
+        system[1].close()
+        mem.append(W.make_system(sc, prec)[1])
+    mem[0].set_spmv_variant(fmt)
+    g = ox.Group(prec)
+    for s in mem:
+        g.add(s)
+    for sc, s in zip(scs, mem):
+        s.set_vector(ox.VEC_UOLD, sc.u0)
+        s.set_vector(ox.VEC_X, sc.u0)
+        W._prepare_step(sc, s, 0, bc, False)
+    g.start(mem, method=method, tol=scs[0].tol, max_iter=30)
+    g.advance(3)
+    assert [s.resident_counts()[0] > 0 for s in mem[1:]] == [not joins] * 2
+    if fmt:
+        assert [s.spmv_format(fp32=prec == ox.FP32_IR) for s in mem[1:]] == [fmt] * 2
+    while g.advance(1000):
+        pass
+    for k in (1, 2):
+        active, info = ox.solve_status(mem[k])
+        _same((mem[k].get_vector(ox.VEC_X), info), refs[k])
+    g.close()
+    for s in mem:
+        s.close()
