@@ -2,6 +2,8 @@
 the launch per phase where it does not or where a resident launch had to leave.
 The counts of the system's resident batches tell them apart, so that a solve
 that quietly took the other way does not pass for one that was tested."""
+import time
+
 import numpy as np
 import pytest
 
@@ -246,3 +248,29 @@ def test_small_members_join_separate_launches(method, bc, prec, fmt, joins):
     g.close()
     for s in mem:
         s.close()
+
+
+@pytest.mark.parametrize("kind,shape,method,bc,prec,max_iter", [
+    # FP64 with x in memory (3 vectors in LDS), and with p there too
+    ("hex", (105, 105, 105), ox.CG, ox.DIRICHLET_SYMMETRIC, ox.FP64, 1500),
+    ("hex", (120, 120, 118), ox.CG, ox.DIRICHLET_SYMMETRIC, ox.FP64, 1000),
+    ("quad", (200, 199), ox.BICGSTAB, ox.DIRICHLET_ROW, ox.FP64, 4500),
+    ("tet", (80, 72, 64), ox.BICGSTAB, ox.DIRICHLET_ROW, ox.FP64, 1500)])
+def test_a_launch_holds_the_chip_for_a_bounded_time(kind, shape, method, bc, prec, max_iter):
+    """No launch takes much more than 10 ms, whatever its system: its iterations
+    go by what one of them costs.  (A tolerance that no solve reaches.)"""
+    sc = _scenario(kind, shape)
+    kw = dict(method=method, dirichlet=bc)
+    system = W.make_system(sc, prec)
+    s = system[1]
+    ref = _solve(sc, system, True, **kw)
+    _same(_solve(sc, system, False, **kw), ref)
+    W._prepare_step(sc, s, 0, bc, False)
+    before = s.resident_counts()[0]
+    t = time.perf_counter()
+    info = s.solve(method=method, tol=1e-300, max_iter=max_iter)
+    t = time.perf_counter() - t
+    run = s.resident_counts()[0] - before
+    print(f"{info['iterations']} iterations, {run} launches, {1e3 * t:.1f} ms")
+    assert run > 1 and t / run < 0.02
+    s.close()
