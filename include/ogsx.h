@@ -114,7 +114,9 @@ int ogsx_pattern_export(const ogsx_pattern* p, int64_t* row_ptr, int64_t* col,
 /* Element colour of every element (n_elem ints). */
 int ogsx_pattern_colors(const ogsx_pattern* p, int32_t* color);
 /* Device bytes that ogsx_system_create + ogsx_system_set_elements (without
- * Gauss-point velocities) allocate for a system on this pattern: what a
+ * Gauss-point velocities) allocate for a system on this pattern, as
+ * ogsx_system_bytes counts it (the driver takes 4.2 MB more for its stream, and
+ * rounds allocations past 1 MiB up to pages of 2 MiB): what a
  * caller that admits work by HBM footprint reserves before creating it.
  * No counterpart in the reference (its matrices live in host memory). */
 int ogsx_pattern_footprint(const ogsx_pattern* p, int precision, int64_t* bytes);
@@ -131,7 +133,7 @@ int ogsx_pattern_destroy(ogsx_pattern* p);
  * diagonal there). */
 int ogsx_system_create(const ogsx_pattern* p, int precision, ogsx_system** out);
 int ogsx_system_destroy(ogsx_system* s);
-/* Device bytes the system has allocated so far. */
+/* Device bytes of the allocations the system has made so far. */
 int ogsx_system_bytes(const ogsx_system* s, int64_t* bytes);
 
 /* Element data for CFiniteElementStd::Assembly (FEM/fem_ele_std.cpp:9367).

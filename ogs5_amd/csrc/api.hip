@@ -141,6 +141,46 @@ struct SolveCtx {
     int seg_key = -1, seg_it0 = 0;
     double seg_e0 = 0.0;
 };
+
+// Arrays share blocks: a release of one array back to the pool costs 11 us, and
+// a system has seventy of them (create, assemble, two solves and destroy on
+// 3,900 rows: 2.95 ms with an allocation per array, 2.11 with the blocks).  A
+// system and its elements of up to kArenaWhole are one block.  In a larger one
+// arrays of kArenaOwn and more have allocations of their own and the others
+// share blocks of kArenaNext, as do all later arrays (larger blocks would waste
+// more to the driver, which rounds what is past 1 MiB up to pages of 2 MiB).
+constexpr size_t kArenaWhole = size_t(8) << 20, kArenaOwn = size_t(1) << 20,
+                 kArenaNext = size_t(256) << 10, kArenaAlign = 256;
+
+size_t arena_room(size_t bytes) { return (bytes + kArenaAlign - 1) & ~(kArenaAlign - 1); }
+
+// Where the arrays go that a system allocates one after the other.
+struct BlockPlan {
+    size_t whole = 0;     // bytes of the first block, where it takes all arrays
+    bool in_whole = false;  // it is the current one
+    size_t left = 0;      // unused bytes of the current block
+    // An array of so many bytes: the block to allocate for it (0: the current
+    // one has room); moves: the rest of that block becomes the current one.
+    size_t take(size_t bytes, bool& moves)
+    {
+        const size_t room = arena_room(bytes);
+        moves = false;
+        if (room <= left && (bytes < kArenaOwn || in_whole)) {
+            left -= room;
+            return 0;
+        }
+        size_t block = bytes < kArenaOwn ? std::max(room, kArenaNext) : bytes;
+        if (whole > 0) block = std::max(room, whole);
+        if (block > room && block - room > left) {
+            left = block - room;
+            moves = true;
+            in_whole = whole > 0;
+        }
+        whole = 0;
+        return block;
+    }
+};
+
 }  // namespace
 
 struct ogsx_system {
@@ -269,9 +309,9 @@ struct ogsx_system {
     size_t ev_next = 0;
     ProfAcc prof_acc[4];
     std::vector<void*> allocs;    // device blocks
-    char* arena = nullptr;        // unused end of one of them, for small arrays
-    size_t arena_left = 0, arena_next = 0;
-    int64_t bytes = 0;  // device bytes of the arrays
+    char* arena = nullptr;        // unused end of one of them
+    BlockPlan plan;
+    int64_t bytes = 0;  // device bytes of the blocks
 };
 
 namespace {
@@ -298,15 +338,6 @@ bool use_pool()
     return pool;
 }
 
-// Arrays of less than kArenaOwn share blocks: a release of one array back to
-// the pool costs 11 us, and a system has seventy of them (create, assemble, two
-// solves and destroy on 3,900 rows: 2.95 ms with an allocation per array, 2.11
-// with the blocks).  The first block takes a whole system of up to kArenaFirst;
-// larger systems and later arrays take blocks of kArenaNext, so that little
-// more than one of those is unused.
-constexpr size_t kArenaOwn = size_t(1) << 20, kArenaFirst = size_t(8) << 20,
-                 kArenaNext = size_t(256) << 10, kArenaAlign = 256;
-
 int block_alloc(ogsx_system* s, char** p, size_t bytes)
 {
     void* q = nullptr;
@@ -314,6 +345,7 @@ int block_alloc(ogsx_system* s, char** p, size_t bytes)
     if (e != hipSuccess)
         return fail(OGSX_ENOMEM, std::string("hipMalloc failed: ") + hipGetErrorString(e));
     s->allocs.push_back(q);
+    s->bytes += (int64_t)bytes;
     *p = (char*)q;
     return OGSX_OK;
 }
@@ -322,22 +354,17 @@ template <typename T>
 int dalloc(ogsx_system* s, T** p, size_t count)
 {
     if (count == 0) count = 1;
-    const size_t bytes = count * sizeof(T), room = (bytes + kArenaAlign - 1) & ~(kArenaAlign - 1);
+    const size_t bytes = count * sizeof(T), room = arena_room(bytes);
+    bool moves = false;
+    const size_t block = s->plan.take(bytes, moves);
     char* q = s->arena;
-    if (bytes < kArenaOwn && room <= s->arena_left) {
-        s->arena += room;
-        s->arena_left -= room;
-    } else {
-        const size_t block = bytes < kArenaOwn ? std::max(room, s->arena_next) : bytes;
+    if (block > 0) {
         const int rc = block_alloc(s, &q, block);
         if (rc != OGSX_OK) return rc;
-        if (bytes < kArenaOwn) s->arena_next = kArenaNext;
-        if (block > room && block - room > s->arena_left) {
-            s->arena = q + room;
-            s->arena_left = block - room;
-        }
+        if (moves) s->arena = q + room;
+    } else {
+        s->arena += room;
     }
-    s->bytes += (int64_t)bytes;
     *p = (T*)q;
     return OGSX_OK;
 }
@@ -727,48 +754,113 @@ void build_layout(const PatternHost& h, PatternLayout& L)
 }
 
 // Device bytes a system on pattern p allocates: ogsx_system_create plus
-// ogsx_system_set_elements without Gauss-point velocities (counted as the
-// allocations ask for them, one element for an empty array).
-int64_t system_bytes(const ogsx_pattern* p, int precision)
+// ogsx_system_set_elements without Gauss-point velocities, array by array in
+// their order.
+struct Footprint {
+    std::vector<size_t> arrays;
+    // `times` arrays of count elements (one element for an empty array)
+    void add(int64_t count, size_t size, int times = 1)
+    {
+        arrays.insert(arrays.end(), times, (size_t)std::max<int64_t>(count, 1) * size);
+    }
+    BlockPlan plan() const
+    {
+        size_t all = 0;
+        for (size_t a : arrays) all += arena_room(a);
+        BlockPlan b;
+        if (all <= kArenaWhole) b.whole = all;
+        return b;
+    }
+    int64_t bytes() const
+    {
+        BlockPlan b = plan();
+        size_t t = 0;
+        bool moves = false;
+        for (size_t a : arrays) t += b.take(a, moves);
+        return (int64_t)t;
+    }
+};
+
+Footprint system_footprint(const ogsx_pattern* p, int precision)
 {
     const PatternHost& h = p->h;
     const PatternLayout& L = p->L;
-    const int64_t n = h.n, nnz = h.nnz, E = h.n_elem, G = grid_for(n);
-    auto b = [](int64_t count, int64_t size) { return std::max<int64_t>(count, 1) * size; };
-    const int ed = edim_of(h.etype);
-    int64_t t = b(n + 1, 4) + b(nnz, 4) + b(n, 4) + b((int64_t)h.conn.size(), 4) +
-                b((int64_t)h.color_elems.size(), 4) + b((int64_t)h.conn.size() * h.npe, 4) + b(nnz, 8) +
-                2 * b(n, 8) + 12 * b(n, 8) + b(16 * (int64_t)part_stride((int)G), 8) +
-                b((int64_t)res_sync_bytes((int)G), 1) + b(8, 8) + b(1, sizeof(KrylovState)) +
-                b(n, 1) + b(n, 8) + b(1, sizeof(SysDev)) + b(1, sizeof(KrylovParams));
-    if (precision == OGSX_FP32_IR) t += b(nnz, 4) + 12 * b(n, 4) + b(n, 8) + b(1, sizeof(IRState));
-    if (!L.sell16)  // tiles and 32-bit SELL columns, built at creation only then
-        t += b((int64_t)L.trow.size(), 4) + b((int64_t)L.tcb.size(), 4) +
-             (L.tile16 ? b((int64_t)L.tc16.size(), 2) : 0) + b((int64_t)L.sc32.size(), 4);
-    t += b((int64_t)L.sptr.size(), 4) + b((int64_t)L.sw.size(), 4) + b((int64_t)L.scb.size(), 4) +
-         b((int64_t)L.ssrc.size(), 4) + b(L.npad, 8) +
-         (precision == OGSX_FP32_IR ? b(L.npad, 4) : 0) + (L.sell16 ? b((int64_t)L.sc16.size(), 2) : 0);
-    if (L.pat_ok) t += b((int64_t)L.spid.size(), 1) + b((int64_t)L.pdelta.size(), 4);
-    if (L.tri_ok) {  // tables, entry map, value arrays sized for the longer layout
-        const int64_t extra = std::max<int64_t>(0, L.npad3 - L.npad);
-        t += b((int64_t)L.tptr.size(), 4) + b((int64_t)L.tid.size(), 2) + b((int64_t)L.tcnt.size(), 4) +
-             b((int64_t)L.toff.size(), 4) + b(L.npad3, 4) + extra * 8 +
-             (precision == OGSX_FP32_IR ? extra * 4 : 0);
+    const int64_t n = h.n, nnz = h.nnz, E = h.n_elem, conn = (int64_t)h.conn.size();
+    const int G = grid_for(n), ed = edim_of(h.etype);
+    const bool ir = precision == OGSX_FP32_IR;
+    Footprint f;
+    f.add(n + 1, 4);
+    f.add(nnz, 4);
+    f.add(n, 4);
+    f.add(conn, 4);
+    f.add((int64_t)h.color_elems.size(), 4);
+    f.add(conn * h.npe, 4);
+    f.add(nnz, 8);
+    f.add(n, 8, 14);  // u_old, IC and the vectors
+    f.add(16 * (int64_t)part_stride(G), 8);
+    f.add((int64_t)res_sync_bytes(G), 1);
+    f.add(8, 8);
+    f.add(1, sizeof(KrylovState));
+    f.add(n, 1);
+    f.add(n, 8);
+    f.add(1, sizeof(SysDev));
+    f.add(1, sizeof(KrylovParams));
+    if (ir) {
+        f.add(nnz, 4);
+        f.add(n, 4, 12);
+        f.add(n, 8);
+        f.add(1, sizeof(IRState));
     }
-    if (L.dia_ok)  // offsets, position map, FP64 values (and FP32 ones for IR)
-        t += b((int64_t)L.doff.size(), 4) + b(((int64_t)L.doff.size() + 1) * n, 4) +
-             b(((int64_t)L.doff.size() + 1) * n, 8) +
-             (precision == OGSX_FP32_IR ? b(((int64_t)L.doff.size() + 1) * n, 4) : 0);
+    f.add((int64_t)L.sptr.size(), 4);
+    f.add((int64_t)L.sw.size(), 4);
+    f.add((int64_t)L.scb.size(), 4);
+    f.add((int64_t)L.ssrc.size(), 4);
+    // value arrays sized for the longer of the SELL and triple layouts
+    const int64_t nval = std::max<int64_t>(L.npad, L.tri_ok ? L.npad3 : 0);
+    f.add(nval, 8);
+    if (ir) f.add(nval, 4);
+    if (L.sell16) f.add((int64_t)L.sc16.size(), 2);
+    if (L.pat_ok) {
+        f.add((int64_t)L.spid.size(), 1);
+        f.add((int64_t)L.pdelta.size(), 4);
+    }
+    if (L.tri_ok) {  // tables, entry map
+        f.add((int64_t)L.tptr.size(), 4);
+        f.add((int64_t)L.tid.size(), 2);
+        f.add((int64_t)L.tcnt.size(), 4);
+        f.add((int64_t)L.toff.size(), 4);
+        f.add((int64_t)L.tsrc.size(), 4);
+    }
+    if (L.dia_ok) {  // offsets, position map, FP64 values (and FP32 ones for IR)
+        const int64_t nd = ((int64_t)L.doff.size() + 1) * n;
+        f.add((int64_t)L.doff.size(), 4);
+        f.add((int64_t)L.dsrc.size(), 4);
+        f.add(nd, 8);
+        if (ir) f.add(nd, 4);
+    }
+    if (!L.sell16) {  // tiles and 32-bit SELL columns, built at creation only then
+        f.add((int64_t)L.trow.size(), 4);
+        f.add((int64_t)L.tcb.size(), 4);
+        if (L.tile16) f.add((int64_t)L.tc16.size(), 2);
+        f.add((int64_t)L.sc32.size(), 4);
+    }
     // element data
-    t += 3 * b(n, 8) + b(E, 8) + b(E * ed * ed, 8) + b(kMaxGaussPts * 8, 8) +
-         b(kMaxGaussPts * 24, 8) + b(kMaxGaussPts * 3, 8);
+    f.add(n, 8, 3);
+    f.add(E, 8);
+    f.add(E * ed * ed, 8);
+    f.add(kMaxGaussPts * 8, 8);
+    f.add(kMaxGaussPts * 24, 8);
+    f.add(kMaxGaussPts * 3, 8);
     // two-pass assembly: incidence, row positions, element matrices and
     // right-hand sides
     if (!h.inc_ptr.empty() && h.row_max <= kAsmRowMax) {
         const int64_t np = h.npe;
-        t += b(n + 1, 4) + 2 * b(E * np, 4) + b(E * np * np, 1) + b(E * np * (np + 2), 8);
+        f.add(n + 1, 4);
+        f.add(E * np, 4, 2);
+        f.add(E * np * np, 1);
+        f.add(E * np * (np + 2), 8);
     }
-    return t;
+    return f;
 }
 
 // ---- profiling helpers ----------------------------------------------------
@@ -1064,7 +1156,7 @@ int ogsx_pattern_footprint(const ogsx_pattern* p, int precision, int64_t* bytes)
 {
     if (!p || !bytes) return fail(OGSX_EINVAL, "null argument");
     if (precision != OGSX_FP64 && precision != OGSX_FP32_IR) return fail(OGSX_EINVAL, "unknown precision");
-    *bytes = system_bytes(p, precision);
+    *bytes = system_footprint(p, precision).bytes();
     return OGSX_OK;
 }
 
@@ -1142,8 +1234,7 @@ int ogsx_system_create(const ogsx_pattern* p, int precision, ogsx_system** out)
         return cleanup(fail(OGSX_EHIP, "hipStreamCreate failed"));
     const PatternHost& h = p->h;
     const PatternLayout& Ly = p->L;
-    const size_t total = (size_t)system_bytes(p, precision);
-    s->arena_next = total <= kArenaFirst ? total + (size_t(64) << 10) : kArenaNext;
+    s->plan = system_footprint(p, precision).plan();
     if ((rc = dalloc(s, &s->ptr, h.n + 1)) || (rc = dalloc(s, &s->col, h.nnz)) ||
         (rc = dalloc(s, &s->diagpos, h.n)) || (rc = dalloc(s, &s->conn, h.conn.size())) ||
         (rc = dalloc(s, &s->color_elems, h.color_elems.size())) ||
