@@ -444,8 +444,8 @@ int ogsx_synchronize(ogsx_system* s);
 int ogsx_resident_counts(ogsx_system* s, int64_t* run, int64_t* left);
 /* Diagnostic: makes the next `batches` resident launches with this system fail.
  * OGSX_RESIDENT_LEAVE: their census waits for one workgroup more than there is,
- * so they leave as on a taken chip.  OGSX_RESIDENT_EXPIRE: their workgroups wait
- * for one another for a single poll; a wait that runs out returns OGSX_EHIP from
+ * so they leave as on a taken chip.  OGSX_RESIDENT_EXPIRE: their workgroups take
+ * their first wait for one another as run out; such a wait returns OGSX_EHIP from
  * the solving call, ends the solves of the launch's systems unconverged, with x
  * undefined, and leaves the systems ready for the next solve.  (A system of one
  * workgroup waits for nobody and does neither.) */

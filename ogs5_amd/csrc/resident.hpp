@@ -92,7 +92,7 @@ struct ResLaunch {
     int entry;
     int wgs;
     int iters;
-    unsigned polls = kResPolls;  // of one wait
+    bool expire = false;  // its first waits count as run out (ogsx_resident_fail)
 };
 
 template <typename T>
@@ -200,7 +200,6 @@ struct ResExchange {
     double (*sw)[4 * VB];  // [kSlotVals] wave sums
     double (*sm)[4];       // [kSlotVals] sums of the waves that poll
     int* ok;
-    unsigned limit;        // polls of one wait
 
     __device__ __forceinline__ OGSX_GL unsigned long long* at(int s, int k, int copy) const
     {
@@ -275,7 +274,9 @@ struct ResExchange {
                     for (int k = 0; k < NV; k++) got[k] = agent_load(at(set, k, w % kSlotCopies) + t);
 #pragma unroll
                     for (int k = 0; k < NV; k++) wait = wait || got[k] == kSlotEmpty;
-                    if (wait && ++polls > limit) {
+                    // (a limit from the launch's arguments: 0.1 us more per
+                    // iteration, the compiler hoists less out of the loop)
+                    if (wait && ++polls > kResPolls) {
                         *ok = 0;
                         break;
                     }
@@ -448,8 +449,8 @@ __global__ __launch_bounds__(kBlock * VB) void k_cg_resident(Grp g, ResLaunch L)
     double ir_error = 0.0, maxr = 0.0;
     double rr = st->rr;
     ResExchange<VB> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, G / VB,
-                       sw, sm, &ok, L.polls};
-    if (tid == 0) ok = 1;
+                       sw, sm, &ok};
+    if (tid == 0) ok = !L.expire;
     if (!res_census(L, idle, &flag)) {
         if (!idle && w == 0 && tid == 0) st->resident = 1;
         return;
@@ -617,8 +618,8 @@ __global__ __launch_bounds__(kBlock * VB) void k_bi_resident(Grp g, ResLaunch L)
     double rho0 = st->rho0, rho1 = st->rho1, alpha_d = st->alpha, omega_d = st->omega;
     double error = st->error;
     ResExchange<VB> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, G / VB,
-                       sw, sm, &ok, L.polls};
-    if (tid == 0) ok = 1;
+                       sw, sm, &ok};
+    if (tid == 0) ok = !L.expire;
     if (!res_census(L, idle, &flag)) {
         if (!idle && w == 0 && tid == 0) st->resident = 1;
         return;
@@ -1268,8 +1269,8 @@ __global__ __launch_bounds__(kBlock * kStreamVb) void k_cg_stream(Grp g, ResLaun
     const double bnorm = st->bnorm;
     const double tol = gl(S.prm)->tol, upd_thresh = gl(S.prm)->upd_thresh;
     double rr = st->rr;
-    ResExchange<VB> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, nwg, sw, sm, &ok, L.polls};
-    if (tid == 0) ok = 1;
+    ResExchange<VB> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, nwg, sw, sm, &ok};
+    if (tid == 0) ok = !L.expire;
     if (!res_census(L, idle, &flag)) {
         if (!idle && w == 0 && tid == 0) st->resident = 1;
         return;
@@ -1489,8 +1490,8 @@ __global__ __launch_bounds__(kBlock * kStreamVb) void k_bi_stream(Grp g, ResLaun
     const double tol = gl(S.prm)->tol;
     double rho0 = st->rho0, rho1 = st->rho1, alpha_d = st->alpha, omega_d = st->omega;
     double error = st->error;
-    ResExchange<VB> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, nwg, sw, sm, &ok, L.polls};
-    if (tid == 0) ok = 1;
+    ResExchange<VB> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, nwg, sw, sm, &ok};
+    if (tid == 0) ok = !L.expire;
     if (!res_census(L, idle, &flag)) {
         if (!idle && w == 0 && tid == 0) st->resident = 1;
         return;

@@ -47,8 +47,8 @@ SEVERAL = [("quad", (200, 199), ox.CG, ox.DIRICHLET_SYMMETRIC),
 @pytest.mark.parametrize("prec", [ox.FP64, ox.FP32_IR])
 @pytest.mark.parametrize("kind,shape,method,bc", SEVERAL)
 def test_an_expired_wait_ends_the_solve(kind, shape, method, bc, prec):
-    """Workgroups that give up waiting at once (every one of them still runs to
-    its end): the call fails, the solve is over and unconverged, and the next one
+    """Workgroups that take their first wait as run out (every one of them still
+    runs to its end): the call fails, the solve is over and unconverged, and the next one
     finds nothing of it."""
     sc = _scenario(kind, shape)
     kw = dict(method=method, dirichlet=bc)
