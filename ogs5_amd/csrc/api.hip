@@ -16,7 +16,6 @@
 #include <string>
 #include <map>
 #include <thread>
-#include <tuple>
 #include <vector>
 
 #include "kernels.hpp"

@@ -600,9 +600,21 @@ __global__ __launch_bounds__(kBlock * VB) void k_cg_resident(Grp g, ResLaunch L)
 // and the p it keeps, so neither needs to be exchanged.  173 x 118 quads
 // (FP64): 9 us per iteration, 24 with five launches; bound by the exchanges
 // (5 us), then by the divisions of a row's columns (exact ones, twice).
+//
+// Five values per entry of a row are more registers than a thread of 512 has for
+// 15 entries in FP64 or 27 in FP32: p and d of the columns are then in LDS.
+template <typename T, int NE, int VB>
+constexpr bool bi_lds()
+{
+    return VB == 2 && NE * sizeof(T) >= 108;
+}
+
 template <typename T, int NE, bool PAIR, int VB>
 __global__ __launch_bounds__(kBlock * VB) void k_bi_resident(Grp g, ResLaunch L)
 {
+    constexpr bool kLds = bi_lds<T, NE, VB>();
+    constexpr int NT = kBlock * VB, NR = kLds ? 1 : NE;
+    extern __shared__ __align__(16) char stream_lds[];
     __shared__ double sw[kSlotVals][4 * VB];
     __shared__ double sm[kSlotVals][4];
     __shared__ int flag, ok;
@@ -630,17 +642,27 @@ __global__ __launch_bounds__(kBlock * VB) void k_bi_resident(Grp g, ResLaunch L)
     const int mine = sb * 64 + tid % kBlock;
     const bool have = mine < min(se * 64, n);
     const int row = have ? mine : n - 1;
-    T a[NE], pj[NE], rj[NE], vj[NE], dj[NE];
+    T a[NE], rj[NE], vj[NE], preg[NR], dreg[NR];
+    T* const pl = (T*)stream_lds + tid;
+    T* const dl = pl + NE * NT;
+    const auto pj = [&](int e) -> T& {
+        if constexpr (kLds) return pl[e * NT];
+        else return preg[e];
+    };
+    const auto dj = [&](int e) -> T& {
+        if constexpr (kLds) return dl[e * NT];
+        else return dreg[e];
+    };
     unsigned col[NE];
     load_row<T, NE, PAIR>(S, sizeof(T) == 8 && gl(S.prm)->dia, row, a, col);
     OGSX_GL T* const rg = wave_uniform(v.r);
     OGSX_GL T* const vg = wave_uniform(v.v);
 #pragma unroll
     for (int e = 0; e < NE; e++) {
-        pj[e] = at_byte(v.p, col[e]);
+        pj(e) = at_byte(v.p, col[e]);
         rj[e] = at_byte(rg, col[e]);
         vj[e] = at_byte(vg, col[e]);
-        dj[e] = at_byte(v.d, col[e]);
+        dj(e) = at_byte(v.d, col[e]);
     }
     auto gather = [&](const OGSX_GL T* from, T (&to)[NE]) {
 #pragma unroll
@@ -678,8 +700,9 @@ __global__ __launch_bounds__(kBlock * VB) void k_bi_resident(Grp g, ResLaunch L)
         T h[NE];  // the preconditioned p, then s, of the row's columns
 #pragma unroll
         for (int e = 0; e < NE; e++) {
-            pj[e] = it == 0 ? rj[e] : bi_p(rj[e], beta, pj[e], omega, vj[e]);
-            h[e] = pj[e] / dj[e];
+            const T pe = it == 0 ? rj[e] : bi_p(rj[e], beta, pj(e), omega, vj[e]);
+            pj(e) = pe;
+            h[e] = pe / dj(e);
         }
         p = it == 0 ? r : bi_p(r, beta, p, omega, vi);
         const T ph = p / d;
@@ -698,7 +721,7 @@ __global__ __launch_bounds__(kBlock * VB) void k_bi_resident(Grp g, ResLaunch L)
 #pragma unroll
         for (int e = 0; e < NE; e++) {
             const T sj = rj[e] - alpha * vj[e];
-            h[e] = sj / dj[e];
+            h[e] = sj / dj(e);
         }
         const T t = row_sum<T, NE, PAIR>(a, h);
         double three[3] = {have ? (double)s * (double)s : 0.0, have ? (double)t * (double)t : 0.0,
