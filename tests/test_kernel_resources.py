@@ -61,7 +61,7 @@ def kernels(ox):
 
 
 # (mangled: template arguments <double, ...>, and the FP64-only kernels)
-NO_ALLOC = [r"k_cg_residentId", r"k_bi_residentId", r"k_cg_oneI", r"k_diag_crs",
+NO_ALLOC = [r"k_cg_residentId", r"k_bi_residentId", r"k_cg_oneI", r"k_bi_oneI", r"k_diag_crs",
             r"k_noalloc_setup", r"k_(cg|bi)_\w*I(Li9E)?dd?", r"k_(cg|bi)_init_final"]
 
 
