@@ -202,6 +202,7 @@ struct ogsx_system {
     size_t tune_n64 = 0;      // leading FP64 entries of tune_log (then FP32)
     bool fmt_default = false;  // fmt64 / fmt32 hold the format of untimed solves
     bool fmt_forced = false;  // formats set by ogsx_set_spmv_variant
+    int fmt_aside = 0;        // the solve's format (IR: FP32) after it, 0: the same
     // SELL-64 copy of the matrix (values refreshed from A when A changed)
     int n_slices = 0;
     int64_t npad = 0;
@@ -2577,6 +2578,7 @@ int ogsx_set_spmv_variant(ogsx_system* s, int lanes_per_row)
 {
     if (!s) return fail(OGSX_EINVAL, "null system");
     if (s->sc.active) return fail(OGSX_ESTATE, "system has a solve in progress");
+    s->fmt_aside = 0;
     if (lanes_per_row == 0) {
         s->fmt64 = s->fmt32 = 0;  // autotune on next use
         s->fmt_forced = s->fmt_default = false;

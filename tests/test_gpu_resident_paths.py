@@ -274,3 +274,27 @@ def test_a_launch_holds_the_chip_for_a_bounded_time(kind, shape, method, bc, pre
     print(f"{info['iterations']} iterations, {run} launches, {1e3 * t:.1f} ms")
     assert run > 1 and t / run < 0.02
     s.close()
+
+
+@pytest.mark.parametrize("prec", [ox.FP64, ox.FP32_IR])
+def test_solves_leave_the_tuned_format(prec):
+    """A streamed BiCGStab solve reads the matrix through the stencil dictionary,
+    whatever the tuner found; after it, and where profiling keeps it to separate
+    launches, the tuner's format is in use."""
+    sc = _scenario("hex", (65, 64, 63))
+    kw = dict(method=ox.BICGSTAB, dirichlet=ox.DIRICHLET_ROW)
+    system = W.make_system(sc, prec)
+    s = system[1]
+
+    def formats():
+        return s.spmv_format(), s.spmv_format(fp32=True)
+
+    ref = _solve(sc, system, True, **kw)
+    tuned = formats()
+    print(f"tuned formats {tuned}")
+    _same(_solve(sc, system, False, **kw), ref)
+    assert s.resident_counts()[0] > 0
+    assert formats() == tuned
+    _same(_solve(sc, system, True, **kw), ref)
+    assert formats() == tuned
+    s.close()
