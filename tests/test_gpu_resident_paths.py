@@ -298,3 +298,36 @@ def test_solves_leave_the_tuned_format(prec):
     _same(_solve(sc, system, True, **kw), ref)
     assert formats() == tuned
     s.close()
+
+
+@pytest.mark.parametrize("prec", [ox.FP64, ox.FP32_IR])
+def test_solves_at_once(prec):
+    """Three solves on their own streams, from threads of their own: a streamed
+    one that takes every compute unit and two of a thread per row, whose launches
+    find the chip taken now and then.  Each gives its own bits every time."""
+    import threading
+    scs = [_scenario("hex", (70, 68, 66)), _scenario("quad", (200, 199)), _scenario("quad", (300, 290))]
+    for sc in scs:
+        sc.max_iter = 120
+    refs, systems = [], []
+    for sc in scs:
+        systems.append(W.make_system(sc, prec))
+        refs.append(_solve(sc, systems[-1], True))
+        systems[-1][1].profile(False)
+    got = [[] for _ in scs]
+
+    def work(k):
+        for _ in range(8):
+            got[k].append(_solve(scs[k], systems[k], False))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    print([s.resident_counts() for _, s in systems])
+    for k in range(3):
+        assert len(got[k]) == 8 and systems[k][1].resident_counts()[0] > 0
+        for r in got[k]:
+            _same(r, refs[k])
+        systems[k][1].close()
