@@ -55,10 +55,12 @@ def gpu_leg(sc, precision, steps, warmup):
     s.synchronize()
     t0 = time.perf_counter()
     infos = []
+    resident = s.resident_counts()[0]
     for _ in range(steps):
         infos.append(run_job(sc, system, precision))
     s.synchronize()
     dt = time.perf_counter() - t0
+    resident = s.resident_counts()[0] - resident
     print(f"[bench] timed precision={precision} steps={steps} {dt:.3f} s", file=sys.stderr,
           flush=True)
     # the same jobs with the node values crossing PCIe (u0 in, x out), as a
@@ -96,6 +98,7 @@ def gpu_leg(sc, precision, steps, warmup):
                             mdof_solves_per_s=solves * sc.n / dt_pcie / 1e6),
         iterations=[i["iterations"] for i in last], outer=[i["outer"] for i in last],
         errors=[i["error"] for i in last],
+        resident_launches_per_step=resident / steps,
         spmv=dict(avg_ms=k_ms, bytes_per_launch=k_bytes, gbs=k_bytes / k_ms / 1e6, launches=50,
                   kernel_alone=True),
         spmv_in_solve=dict(avg_ms=spmv_in_ms, launches=launches, bytes_per_launch=bpl,
@@ -717,6 +720,12 @@ def main():
                 # of one untimed job): p is rewritten between launches
                 frac_in_solve=alg / in_ms / 1e6 / peak if in_ms else None,
                 avg_launch_ms_in_solve=in_ms)
+    if best["resident_launches_per_step"]:
+        # the timed jobs' iterations run in resident launches, which profiling
+        # keeps out of: the matrix and vector bytes above once per iteration over
+        # the whole job's time, a lower bound on the rate of those launches
+        gbs = alg * sum(best["iterations"]) / best["ms_per_step"] / 1e6
+        roof.update(timed_kernel="k_cg_stream", timed_gbs=gbs, timed_frac=gbs / peak)
     # HBM bytes per dispatch of this kernel and format, from the FETCH_SIZE /
     # WRITE_SIZE passes over `bench.py --mode spmv` (profiles/spmv_hex128_traffic.md)
     tf = os.path.join(ROOT, "profiles", "traffic.json")

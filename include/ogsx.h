@@ -352,7 +352,10 @@ int ogsx_solve_crs_noalloc(int64_t n, const int32_t* row_ptr_dev, const int32_t*
 /* Enables HIP-event timing of every SpMV launch that ogsx_solve issues, of
  * ogsx_assemble and of ogsx_gauss_velocity (on the system's stream) and
  * returns the running totals; bytes_per_launch is the kernel's algorithmic
- * HBM traffic per launch (SpMV, velocity; 0 for the assembly). */
+ * HBM traffic per launch (SpMV, velocity; 0 for the assembly).  While it is on
+ * the solves of a system alone take a launch per Krylov phase, not resident
+ * launches, which have no SpMV launch to time: the totals describe those
+ * kernels, and the solve takes their time (the results are the same). */
 int ogsx_profile_enable(ogsx_system* s, int on);
 int ogsx_profile_read(ogsx_system* s, int kind, double* total_ms,
                       int64_t* launches, double* bytes_per_launch);
