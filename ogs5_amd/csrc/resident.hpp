@@ -193,7 +193,7 @@ __device__ __forceinline__ bool res_census(const ResLaunch& L, bool idle, int* f
 
 // Exchange of NV dot products among the workgroups of one system (VB chunks
 // of 256 threads each per workgroup, q chunks to a slot).
-template <int VB>
+template <int VB, bool STREAM = false>
 struct ResExchange {
     OGSX_GL unsigned long long* slot;
     int slots, q, w, set, nwg;
@@ -266,7 +266,8 @@ struct ResExchange {
 #pragma unroll
             for (int k = 0; k < NV; k++) got[k] = 0;
             if (t < nwg * per) {
-                unsigned polls = 0;
+                unsigned polls = 0, limit = kResPolls;
+                if constexpr (STREAM) asm("" : "+s"(limit));
 #pragma nounroll
                 for (bool wait = true; wait;) {
                     wait = false;
@@ -274,9 +275,11 @@ struct ResExchange {
                     for (int k = 0; k < NV; k++) got[k] = agent_load(at(set, k, w % kSlotCopies) + t);
 #pragma unroll
                     for (int k = 0; k < NV; k++) wait = wait || got[k] == kSlotEmpty;
-                    // (a limit from the launch's arguments: 0.1 us more per
-                    // iteration, the compiler hoists less out of the loop)
-                    if (wait && ++polls > kResPolls) {
+                    // (a constant the compiler sees in the thread-per-row kernels,
+                    // one it does not in the streaming ones: it hoists more out
+                    // of the loop with the first, 0.1 us per iteration faster in
+                    // those and 0.7 us slower, by its spills, in these)
+                    if (wait && ++polls > limit) {
                         *ok = 0;
                         break;
                     }
@@ -1292,7 +1295,7 @@ __global__ __launch_bounds__(kBlock * kStreamVb) void k_cg_stream(Grp g, ResLaun
     const double bnorm = st->bnorm;
     const double tol = gl(S.prm)->tol, upd_thresh = gl(S.prm)->upd_thresh;
     double rr = st->rr;
-    ResExchange<VB> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, nwg, sw, sm, &ok};
+    ResExchange<VB, true> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, nwg, sw, sm, &ok};
     if (tid == 0) ok = !L.expire;
     if (!res_census(L, idle, &flag)) {
         if (!idle && w == 0 && tid == 0) st->resident = 1;
@@ -1513,7 +1516,7 @@ __global__ __launch_bounds__(kBlock * kStreamVb) void k_bi_stream(Grp g, ResLaun
     const double tol = gl(S.prm)->tol;
     double rho0 = st->rho0, rho1 = st->rho1, alpha_d = st->alpha, omega_d = st->omega;
     double error = st->error;
-    ResExchange<VB> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, nwg, sw, sm, &ok};
+    ResExchange<VB, true> ex{gl(S.rs->slot), res_slots(G), part_q(G), w, S.rs->phase, nwg, sw, sm, &ok};
     if (tid == 0) ok = !L.expire;
     if (!res_census(L, idle, &flag)) {
         if (!idle && w == 0 && tid == 0) st->resident = 1;
