@@ -601,7 +601,7 @@ __global__ __launch_bounds__(kBlock * VB) void k_cg_resident(Grp g, ResLaunch L)
 //   (r, r), (r0, r), with r published.
 // A thread forms p and s of its columns itself, from the r and v it gathers
 // and the p it keeps, so neither needs to be exchanged.  173 x 118 quads
-// (FP64): 9 us per iteration, 24 with five launches; bound by the exchanges
+// (FP64): 8 us per iteration, 24 with five launches; bound by the exchanges
 // (5 us), then by the divisions of a row's columns (exact ones, twice).
 //
 // Five values per entry of a row are more registers than a thread of 512 has for
